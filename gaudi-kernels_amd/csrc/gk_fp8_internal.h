@@ -241,6 +241,8 @@ struct GemmArgs {
 hipError_t launch_gemm_decode(const GemmArgs& a, hipStream_t stream);
 hipError_t launch_gemm_prefill(const GemmArgs& a, hipStream_t stream);     // dispatches by M
 hipError_t launch_gemm_prefill256(const GemmArgs& a, hipStream_t stream);  // 256 x 256 tiles, Mpad % 256 == 0
+// Smaller tiles of the same GEMM (gk_fp8_tiles.hip): the same conditions, the same result bits.  Also the channel form.
+hipError_t launch_gemm_tiles(const GemmArgs& a, TileId tile, hipStream_t stream);
 // The 256 x 256 kernels address a 256-row weight panel and the whole
 // group-major activation array with 32-bit byte offsets.
 inline bool prefill256_fits(const GemmArgs& a) {

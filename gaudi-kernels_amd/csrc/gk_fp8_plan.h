@@ -107,4 +107,70 @@ constexpr int dense_tile_of(int bid, int tiles_m, int tiles_nn, int kparts) {
   return (sb * 4 + rem % wsb) * 65536 + rem / wsb;
 }
 
+// Columns [0, n_wide) in 256-wide weight tiles and the rest in 192-wide tiles,
+// when that fills the CUs better than 256-wide tiles alone: a GEMM whose
+// 256 x 256 tiles need more than one round over the CUs otherwise leaves CUs
+// idle in its last round (M = 4096, N = 7168: 448 tiles on 256 CUs = 1.75
+// rounds, run as 256 + 256 tiles of 256 and 192 columns).  Work is counted in
+// rounds, a 192-wide tile taking 0.8 of a 256-wide one (it keeps the activation
+// traffic of the full tile).  Returns N (no split) when nothing gains; *rounds
+// is the estimate of what is returned.
+inline int prefill_wide_columns(int Mpad, int N, int cus, double* rounds_out = nullptr) {
+  const long long tiles_m = Mpad / 256;
+  const int nt = static_cast<int>((N + 255LL) / 256);
+  auto rounds = [cus](long long tiles) { return static_cast<double>((tiles + cus - 1) / cus); };
+  double best = cus > 0 ? rounds(tiles_m * nt) : 1.0;
+  int best_wide = N;
+  if (cus > 0 && tiles_m * nt > cus) {
+    for (int a = 1; a < nt; ++a) {
+      const int n2 = N - 256 * a;
+      const double est = rounds(tiles_m * a) + 0.8 * rounds(tiles_m * ((n2 + 191LL) / 192)) + 0.02;
+      if (est < best - 1e-9) {
+        best = est;
+        best_wide = 256 * a;
+      }
+    }
+  }
+  if (rounds_out) *rounds_out = best;
+  return best_wide;
+}
+
+// Tile of the LDS-tiled FP8 GEMM (weight rows x tokens).  kTile128x64Two keeps
+// the LDS of two workgroups on a CU (shorter stages), the others use it whole.
+enum TileId { kTile64x32 = 0, kTile64x64, kTile128x64, kTile128x64Two, kTile128x128, kTile256 };
+
+// Which tile: the least estimated time, rounds over the CUs times the time of
+// one 128-K group in a round.  That time, measured on MI355X (us a group and
+// round; bits are the same for every tile): 64 x 32 0.27, 64 x 64 0.29, 128 x 64
+// 0.46, 128 x 128 0.73, 256 x 256 1.42 on an almost empty chip and 1.66 with all
+// CUs busy; with two workgroups on a CU 128 x 64 0.40 a tile.
+// M = 300, N = 6144, K = 4096: 49.8 us in 48 tiles of 256 x 256, 18.2 us in 240
+// tiles of 128 x 64; M = 1024, N = K = 4096: 49.2 and 26.4 us (128 x 128); M =
+// 1024, N = 28672: 143 us in 256 x 256 tiles, 172 us in 128 x 128 ones.
+inline TileId plan_tile(int M, int Mpad, int N, int cus) {
+  if (cus <= 0) return kTile256;
+  auto rounds = [&](long long bn, long long bm) {
+    const long long tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    return static_cast<double>((tiles + cus - 1) / cus);
+  };
+  double best = 0.0;
+  prefill_wide_columns(Mpad, N, cus, &best);
+  const double tiles256 = static_cast<double>(Mpad / 256) * ((N + 255LL) / 256);
+  best *= 1.42 + 0.24 * (tiles256 < cus ? tiles256 / cus : 1.0);
+  TileId id = kTile256;
+  auto offer = [&](TileId t, double cost) {
+    if (cost < best) {
+      best = cost;
+      id = t;
+    }
+  };
+  const double r6432 = rounds(64, 32), r6464 = rounds(64, 64), r12864 = rounds(128, 64);
+  offer(kTile128x128, 0.73 * rounds(128, 128));
+  if (r12864 <= 1.0) offer(kTile128x64, 0.46);
+  else offer(kTile128x64Two, 0.40 * r12864);
+  offer(kTile64x64, 0.29 * r6464);
+  offer(kTile64x32, 0.27 * r6432);
+  return id;
+}
+
 }  // namespace gk

@@ -801,31 +801,6 @@ hipError_t launch_dense(const GemmArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-// Columns [0, n_wide) in 256-wide weight tiles and the rest in 192-wide tiles,
-// when that fills the CUs better than 256-wide tiles alone: a GEMM whose
-// 256 x 256 tiles need more than one round over the CUs otherwise leaves CUs
-// idle in its last round (config 4: 448 tiles on 256 CUs = 1.75 rounds, run
-// as 256 + 256 tiles of 256 and 192 columns).  Work is counted in rounds, a
-// 192-wide tile taking 0.8 of a 256-wide one (it keeps the activation
-// traffic of the full tile).  Returns N (no split) when nothing gains.
-int prefill_wide_columns(int Mpad, int N, int cus) {
-  const int tiles_m = Mpad / kBM;
-  const int nt = (N + 255) / 256;
-  if (cus <= 0 || tiles_m * nt <= cus) return N;
-  auto rounds = [cus](int tiles) { return (tiles + cus - 1) / cus; };
-  double best = rounds(tiles_m * nt);
-  int best_wide = N;
-  for (int a = 1; a < nt; ++a) {
-    const int n2 = N - 256 * a;
-    const double est = rounds(tiles_m * a) + 0.8 * rounds(tiles_m * ((n2 + 191) / 192)) + 0.02;
-    if (est < best - 1e-9) {
-      best = est;
-      best_wide = 256 * a;
-    }
-  }
-  return best_wide;
-}
-
 // Per-token / per-channel form: a.qa row-major [M][a.ldq], a.sa [M], a.sw [N]; any M.
 hipError_t launch_gemm_channel256(const GemmArgs& a, hipStream_t stream) {
   if (static_cast<int64_t>(256) * a.ldq > int64_t{0xffffffff} || static_cast<int64_t>(256) * a.K > int64_t{0xffffffff})
@@ -841,12 +816,15 @@ hipError_t launch_gemm_channel256(const GemmArgs& a, hipStream_t stream) {
 }
 
 // Requires K % 128 == 0, 16-byte aligned weights, Mpad % 256 == 0 (qa/sa
-// padded with zero rows up to Mpad).  Large GEMMs may run in two column
+// padded with zero rows up to Mpad).  Shapes that 256 x 256 tiles would spread
+// over too few CUs run smaller tiles (plan_tile, gk_fp8_tiles.hip).  Large GEMMs may run in two column
 // ranges of different tile widths (prefill_wide_columns), in one launch; each
 // output column is computed by one workgroup either way, with the same
 // per-element arithmetic.
 hipError_t launch_gemm_prefill256(const GemmArgs& a, hipStream_t stream) {
   if (a.Mpad % kBM != 0 || !prefill256_fits(a)) return hipErrorInvalidValue;
+  const TileId tile = plan_tile(a.M, a.Mpad, a.N, device_cus());
+  if (tile != kTile256) return launch_gemm_tiles(a, tile, stream);
   const int wide = prefill_wide_columns(a.Mpad, a.N, device_cus());
   if (wide >= a.N) return launch_dense<4>(a, stream);
   if (a.wpack) return a.half_w ? launch_split<true, true>(a, wide, stream) : launch_split<false, true>(a, wide, stream);
