@@ -323,33 +323,149 @@ __global__ __launch_bounds__(NW * 64) void gemm_decode_kernel(const uint8_t* __r
 }
 
 // ---------------------------------------------------------------------------
-// Generic variant for shapes the tiled kernels do not take (K % 128 != 0 or
-// misaligned weights): one thread per output, byte loads with K bounds.
-__global__ __launch_bounds__(256) void gemm_generic_kernel(const uint8_t* __restrict__ qa,
-                                                           const float* __restrict__ sa,
-                                                           const uint8_t* __restrict__ w,
-                                                           const float* __restrict__ sw,
-                                                           const float* __restrict__ bias,
-                                                           uint16_t* __restrict__ y, int64_t ldy, int M, int N,
-                                                           int K, int G, int Mpad, int half_w) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (idx >= static_cast<int64_t>(M) * N) return;
-  const int m = static_cast<int>(idx / N), n = static_cast<int>(idx % N);
-  float acc = 0.0f;
-  for (int g = 0; g < G; ++g) {
-    float part = 0.0f;
-    const int kend = min(128, K - g * 128);
-    for (int i = 0; i < kend; ++i) {
-      const int64_t k = static_cast<int64_t>(g) * 128 + i;
-      uint32_t wc = w[static_cast<int64_t>(n) * K + k];
-      if (half_w) wc = codec_half4(wc) & 0xffu;
-      part = fmaf(e4m3_value(qa[(static_cast<int64_t>(g) * Mpad + m) * 128 + i]), e4m3_value(wc), part);
+// Generic variant for shapes the tiled kernels do not take (K % 128 != 0,
+// weights that are not 16-byte aligned, panels past 32-bit offsets).
+//
+// The E4M3 codes are widened to bf16 (exact: four significant bits) and
+// multiplied by v_mfma_f32_16x16x32_bf16, whose products are exact and whose
+// sums are fp32: the accuracy of the fp32 dot products that this variant
+// computed one output per thread (error against 64 bits, M = 200, N = K = 2880,
+// 1.7e-3 before and after, the bf16 rounding of y; the FP8 matrix
+// instruction's own sums are coarser, 3e-5).  One 128-K group of a 16 x 16 block
+// is four of them; the group's sum takes its scales as in the other variants.
+//
+// Workgroup = kGW waves over 32 weight rows x 16 MB tokens, the groups dealt
+// round-robin to the waves; the kGW partial tiles are summed in wave order.  A
+// wave stages its group in its own LDS (no barrier in the loop): 16-byte weight
+// loads at any byte alignment, or single bytes where a row's last chunk would
+// pass K (those past K become zero), the next group's loads in flight during the
+// current one's products.  Bound by the latency of a wave's few load rounds, so
+// the tile is small and K is split: M = 200, N = K = 2880 7.0 ms (byte loads, one
+// output a thread) -> 19.4 us.
+constexpr int kGW = 8;
+
+// 8 E4M3 codes -> 8 bf16 values.
+__device__ inline bf16x8 widen8(uint32_t lo, uint32_t hi) {
+  const bf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false);
+  const bf16x2 b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true);
+  const bf16x2 c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false);
+  const bf16x2 d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true);
+  return bf16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+
+template <int MB, bool HALF>
+__global__ __launch_bounds__(64 * kGW) void gemm_generic_kernel(const uint8_t* __restrict__ qa,
+                                                                const float* __restrict__ sa,
+                                                                const uint8_t* __restrict__ w,
+                                                                const float* __restrict__ sw,
+                                                                const float* __restrict__ bias,
+                                                                uint16_t* __restrict__ y, int64_t ldy, int M, int N,
+                                                                int K, int G, int Mpad, int tiles_m) {
+  constexpr int NA = 2, kWaveLds = (16 * NA + 16 * MB) * 128;
+  static_assert(kWaveLds >= NA * MB * 64 * 16, "the partial tile fits the wave's staging buffer");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kGW][kWaveLds];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int n0 = static_cast<int>(blockIdx.x / tiles_m) * 16 * NA, m0 = static_cast<int>(blockIdx.x % tiles_m) * 16 * MB;
+  const int lr = lane >> 3, lc = lane & 7;  // loader: row lr of each 8-row piece, 16-byte chunk lc
+  const uint8_t* wrow[2 * NA];
+  const uint8_t* arow[2 * MB];
+#pragma unroll
+  for (int i = 0; i < 2 * NA; ++i) wrow[i] = w + static_cast<int64_t>(min(n0 + 8 * i + lr, N - 1)) * K + 16 * lc;
+#pragma unroll
+  for (int i = 0; i < 2 * MB; ++i) arow[i] = qa + static_cast<int64_t>(min(m0 + 8 * i + lr, M - 1)) * 128 + 16 * lc;
+  u32x4 wr[2 * NA], ar[2 * MB];
+  auto load = [&](int g) {
+    const int left = K - (g * 128 + 16 * lc);  // bytes of the row from this chunk on
+#pragma unroll
+    for (int i = 0; i < 2 * NA; ++i) {
+      const uint8_t* p = wrow[i] + static_cast<int64_t>(g) * 128;
+      if (left >= 16) {
+        __builtin_memcpy(&wr[i], p, 16);
+      } else {
+        uint32_t v[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (e < left) v[e >> 2] |= static_cast<uint32_t>(p[e]) << (8 * (e & 3));
+        wr[i] = u32x4{v[0], v[1], v[2], v[3]};
+      }
     }
-    const float swg = sw[static_cast<int64_t>(n >> 7) * G + g];
-    acc = fmaf(part, sa[static_cast<int64_t>(g) * Mpad + m] * (half_w ? 2.0f * swg : swg), acc);
+#pragma unroll
+    for (int i = 0; i < 2 * MB; ++i)
+      ar[i] = *reinterpret_cast<const u32x4*>(arow[i] + static_cast<int64_t>(g) * Mpad * 128);
+  };
+
+  const int fr = lane & 15, fq = lane >> 4;
+  const uint32_t x0 = ((2 * fq) ^ lds_key(fr)) << 4, x1 = ((2 * fq + 1) ^ lds_key(fr)) << 4;
+  uint8_t* wl = lds[wave];
+  uint8_t* al = wl + 16 * NA * 128;
+  const float* swp = sw + static_cast<int64_t>(n0 >> 7) * G;  // 32 rows at a multiple of 32: one scale block
+  const float* sap[MB];
+#pragma unroll
+  for (int j = 0; j < MB; ++j) sap[j] = sa + min(m0 + 16 * j + fr, M - 1);
+  v4f acc[NA][MB];
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+#pragma unroll
+    for (int j = 0; j < MB; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  if (wave < G) load(wave);
+  for (int g = wave; g < G; g += kGW) {
+    float f[MB];
+#pragma unroll
+    for (int j = 0; j < MB; ++j) {
+      const float ws = swp[g];
+      f[j] = sap[j][static_cast<int64_t>(g) * Mpad] * (HALF ? 2.0f * ws : ws);
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * NA; ++i) {
+      u32x4 v = wr[i];
+      if (HALF) v = u32x4{codec_half4(v[0]), codec_half4(v[1]), codec_half4(v[2]), codec_half4(v[3])};
+      const int r = 8 * i + lr;
+      *reinterpret_cast<u32x4*>(wl + r * 128 + ((lc ^ lds_key(r)) << 4)) = v;
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * MB; ++i) {
+      const int r = 8 * i + lr;
+      *reinterpret_cast<u32x4*>(al + r * 128 + ((lc ^ lds_key(r)) << 4)) = ar[i];
+    }
+    if (g + kGW < G) load(g + kGW);
+    // fragments: lane -> row lane % 16, K bytes [32 (lane / 16), +32); product s takes bytes [8 s, 8 s + 8) of
+    // those on both sides, so together the four cover the group once
+    bf16x8 b[MB][4];
+#pragma unroll
+    for (int j = 0; j < MB; ++j) {
+      const u32x4 lo = *reinterpret_cast<const u32x4*>(al + (16 * j + fr) * 128 + x0);
+      const u32x4 hi = *reinterpret_cast<const u32x4*>(al + (16 * j + fr) * 128 + x1);
+      b[j][0] = widen8(lo[0], lo[1]); b[j][1] = widen8(lo[2], lo[3]);
+      b[j][2] = widen8(hi[0], hi[1]); b[j][3] = widen8(hi[2], hi[3]);
+    }
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      const u32x4 lo = *reinterpret_cast<const u32x4*>(wl + (16 * i + fr) * 128 + x0);
+      const u32x4 hi = *reinterpret_cast<const u32x4*>(wl + (16 * i + fr) * 128 + x1);
+      const bf16x8 a[4] = {widen8(lo[0], lo[1]), widen8(lo[2], lo[3]), widen8(hi[0], hi[1]), widen8(hi[2], hi[3])};
+#pragma unroll
+      for (int j = 0; j < MB; ++j) {
+        v4f t = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], b[j][s], t, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaf(t[r], f[j], acc[i][j][r]);
+      }
+    }
   }
-  if (bias) acc += bias[n];
-  y[static_cast<int64_t>(m) * ldy + n] = bf16_rne(acc);
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+#pragma unroll
+    for (int j = 0; j < MB; ++j) *reinterpret_cast<v4f*>(wl + (i * MB + j) * 1024 + lane * 16) = acc[i][j];
+  __syncthreads();
+  // wave t sums block t of the kGW partial tiles in wave order
+  for (int t = wave; t < NA * MB; t += kGW) {
+    v4f sum = *reinterpret_cast<const v4f*>(lds[0] + t * 1024 + lane * 16);
+#pragma unroll
+    for (int v = 1; v < kGW; ++v) sum += *reinterpret_cast<const v4f*>(lds[v] + t * 1024 + lane * 16);
+    store_tile(y, ldy, bias, M, N, m0 + 16 * (t % MB) + fr, n0 + 16 * (t / MB) + 4 * fq, sum);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -441,12 +557,22 @@ hipError_t launch_gemm_token_channel(const GemmArgs& a, hipStream_t stream) {
   }
 }
 
-hipError_t launch_gemm_generic(const GemmArgs& a, hipStream_t stream) {
-  const int64_t total = static_cast<int64_t>(a.M) * a.N;
-  const dim3 grid(static_cast<unsigned>((total + 255) / 256));
-  gemm_generic_kernel<<<grid, 256, 0, stream>>>(a.qa, a.sa, a.w, a.sw, a.bias, a.y, a.ldy, a.M, a.N, a.K, a.G,
-                                                a.Mpad, a.half_w ? 1 : 0);
+template <int MB>
+static hipError_t generic_launch(const GemmArgs& a, hipStream_t stream) {
+  const int64_t tiles_m = (a.M + 16 * MB - 1LL) / (16 * MB), tiles = tiles_m * ((a.N + 31LL) / 32);
+  if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
+  if (a.half_w)
+    gemm_generic_kernel<MB, true><<<static_cast<unsigned>(tiles), 64 * kGW, 0, stream>>>(
+        a.qa, a.sa, a.w, a.sw, a.bias, a.y, a.ldy, a.M, a.N, a.K, a.G, a.Mpad, static_cast<int>(tiles_m));
+  else
+    gemm_generic_kernel<MB, false><<<static_cast<unsigned>(tiles), 64 * kGW, 0, stream>>>(
+        a.qa, a.sa, a.w, a.sw, a.bias, a.y, a.ldy, a.M, a.N, a.K, a.G, a.Mpad, static_cast<int>(tiles_m));
   return hipGetLastError();
+}
+
+hipError_t launch_gemm_generic(const GemmArgs& a, hipStream_t stream) {
+  // up to 16 tokens fill one block; beyond, two share each weight fragment
+  return a.M <= 16 ? generic_launch<1>(a, stream) : generic_launch<2>(a, stream);
 }
 
 }  // namespace gk

@@ -7,6 +7,7 @@
 namespace gk {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // Chunk key of tile row r: the 16-byte chunk c of row r sits at slot
 // c ^ lds_key(r) of its 128-byte LDS row.  Bits 3, 1, 2 of r give bits 2, 1,
