@@ -17,6 +17,8 @@
 // the IEEE quotient (quant_group8 in gk_fp8_internal.h).  Sixteen lanes own
 // one group (8 bf16 each, one 16-byte load per lane).
 
+#include <algorithm>
+
 #include "gk_fp8_internal.h"
 
 namespace gk {
@@ -62,11 +64,38 @@ __device__ inline void block_status(uint32_t count, uint32_t bad, uint32_t flag_
   }
 }
 
+// Scales: forward doubles, inverse halves; both validate (finite, >= 0).
+// Folded into the byte kernels: a kernel of its own took 6.3-8 us for the 7168
+// scales of a 28672 x 4096 weight (one dependent load and atomic a wave).
+template <bool FORWARD>
+__device__ inline void codec_scales(const float* __restrict__ s, float* __restrict__ out, int64_t n,
+                                    uint32_t* __restrict__ flags) {
+  uint32_t f = 0;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const float v = s[i];
+    const uint32_t b = f32_bits(v);
+    if (!(v >= 0.0f) || (b & 0x7f800000u) == 0x7f800000u) f |= kFlagBadScale;  // NaN, inf, negative
+    if (FORWARD) {
+      const float d = v * 2.0f;
+      if ((f32_bits(d) & 0x7f800000u) == 0x7f800000u) f |= kFlagScaleOverflow;
+      out[i] = d;
+    } else {
+      if ((b & 0x7f800000u) <= 0x00800000u && (b & 1u)) f |= kFlagInexactHalve;
+      out[i] = v * 0.5f;
+    }
+  }
+  if (f) atomicOr(flags, f);  // only on an error
+}
+
 template <bool FORWARD>
 __global__ __launch_bounds__(256) void codec_bytes_kernel(const uint8_t* __restrict__ src,
                                                           uint8_t* __restrict__ dst, int64_t n,
+                                                          const float* __restrict__ scales,
+                                                          float* __restrict__ scales_out, int64_t n_scales,
                                                           uint32_t* __restrict__ flags,
                                                           unsigned long long* __restrict__ rounded) {
+  codec_scales<FORWARD>(scales, scales_out, n_scales, flags);
   const int64_t nvec = n >> 4;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   const int64_t tid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -117,8 +146,11 @@ __global__ __launch_bounds__(256) void codec_bytes_kernel(const uint8_t* __restr
 template <bool FORWARD>
 __global__ __launch_bounds__(256) void codec_unaligned_kernel(const uint8_t* __restrict__ src,
                                                               uint8_t* __restrict__ dst, int64_t n,
+                                                              const float* __restrict__ scales,
+                                                              float* __restrict__ scales_out, int64_t n_scales,
                                                               uint32_t* __restrict__ flags,
                                                               unsigned long long* __restrict__ rounded) {
+  codec_scales<FORWARD>(scales, scales_out, n_scales, flags);
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   uint32_t bad = 0, count = 0;
   for (int64_t j = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; j < n; j += stride) {
@@ -133,29 +165,6 @@ __global__ __launch_bounds__(256) void codec_unaligned_kernel(const uint8_t* __r
     }
   }
   block_status(count, bad, FORWARD ? kFlagNanCode : kFlagInvalidHalf, flags, rounded);
-}
-
-// Scales: forward doubles, inverse halves; both validate (finite, >= 0).
-template <bool FORWARD>
-__global__ __launch_bounds__(256) void codec_scales_kernel(const float* __restrict__ s, float* __restrict__ out,
-                                                           int64_t n, uint32_t* __restrict__ flags) {
-  uint32_t f = 0;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const float v = s[i];
-    const uint32_t b = f32_bits(v);
-    if (!(v >= 0.0f) || (b & 0x7f800000u) == 0x7f800000u) f |= kFlagBadScale;  // NaN, inf, negative
-    if (FORWARD) {
-      const float d = v * 2.0f;
-      if ((f32_bits(d) & 0x7f800000u) == 0x7f800000u) f |= kFlagScaleOverflow;
-      out[i] = d;
-    } else {
-      if ((b & 0x7f800000u) <= 0x00800000u && (b & 1u)) f |= kFlagInexactHalve;
-      out[i] = v * 0.5f;
-    }
-  }
-  f = wave_or_u32(f);
-  if ((threadIdx.x & 63) == 0 && f) atomicOr(flags, f);
 }
 
 // ---- activation quantizer ----------------------------------------------------
@@ -264,30 +273,19 @@ hipError_t launch_codec(bool forward, const uint8_t* src, uint8_t* dst, int64_t 
                         float* scales_out, int64_t n_scales, uint32_t* flags, unsigned long long* rounded,
                         hipStream_t stream) {
   const bool vec = ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0;
+  // 4 workgroups a CU, grid-stride over the codes and the scales
+  const int blocks = std::min(1024, std::max(codec_grid(vec ? n >> 4 : n), codec_grid(n_scales)));
+#define GK_CODEC(KERNEL, F) \
+  KERNEL<F><<<blocks, 256, 0, stream>>>(src, dst, n, scales, scales_out, n_scales, flags, rounded)
   if (vec) {
-    const int blocks = codec_grid(n >> 4) < 1024 ? codec_grid(n >> 4) : 1024;  // 4 per CU, grid-stride
-    if (forward)
-      codec_bytes_kernel<true><<<blocks, 256, 0, stream>>>(src, dst, n, flags, rounded);
-    else
-      codec_bytes_kernel<false><<<blocks, 256, 0, stream>>>(src, dst, n, flags, rounded);
+    if (forward) GK_CODEC(codec_bytes_kernel, true);
+    else GK_CODEC(codec_bytes_kernel, false);
   } else {
-    const int blocks = codec_grid(n) < 1024 ? codec_grid(n) : 1024;
-    if (forward)
-      codec_unaligned_kernel<true><<<blocks, 256, 0, stream>>>(src, dst, n, flags, rounded);
-    else
-      codec_unaligned_kernel<false><<<blocks, 256, 0, stream>>>(src, dst, n, flags, rounded);
+    if (forward) GK_CODEC(codec_unaligned_kernel, true);
+    else GK_CODEC(codec_unaligned_kernel, false);
   }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  if (n_scales > 0) {
-    const int sblocks = codec_grid(n_scales / 16 + 1);
-    if (forward)
-      codec_scales_kernel<true><<<sblocks, 256, 0, stream>>>(scales, scales_out, n_scales, flags);
-    else
-      codec_scales_kernel<false><<<sblocks, 256, 0, stream>>>(scales, scales_out, n_scales, flags);
-    e = hipGetLastError();
-  }
-  return e;
+#undef GK_CODEC
+  return hipGetLastError();
 }
 
 hipError_t launch_pack_weight(const uint8_t* w, int N, int K, uint8_t* packed, hipStream_t stream) {
