@@ -566,27 +566,7 @@ __device__ __forceinline__ void prefill256_body(int block, const uint8_t* __rest
     return;
   }
 
-  if (CH) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (j < jl) {
-        const int m = m0 + mw + j * kJS + fr;
-        if (m < M) {
-          const float sam = sa[m];
-          uint16_t* row = y + static_cast<int64_t>(m) * ldy;
-#pragma unroll
-          for (int i = 0; i < NA; ++i) {
-            const int n = n0 + wn * 16 * NA + i * 16 + 4 * fq;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (n + r < N) row[n + r] = channel_out(acc[i][j][r], sam, sw[n + r], bias ? bias[n + r] : 0.0f);
-          }
-        }
-      }
-    }
-    return;
-  }
-  if (yp) {
+  if (!CH && yp) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       if (j < jl) {
@@ -615,24 +595,34 @@ __device__ __forceinline__ void prefill256_body(int block, const uint8_t* __rest
     // a stride of BN * 2 + 16, then whole-row 16-byte stores.  The fragment
     // layout would store 32-byte pieces of 16 rows per instruction; every
     // workgroup of a round stores its tile at once, so the epilogue is a
-    // write burst (measured on MI355X, config 4 GEMM: -1%).  Same bits as
-    // store_tile: bias added in fp32, one bf16 rounding.
+    // write burst (measured on MI355X, config 4 GEMM: -1%; the channel form,
+    // which stored single values: M = 2048, N = 7168, K = 4096 101 -> 68 us).
+    // Same bits as store_tile and channel_out: fp32, one bf16 rounding.
     constexpr int kRS = BN * 2 + 16, kCPR = BN / 8;  // LDS row stride; 16-byte chunks per row
     static_assert(kBM * kRS <= kLdsBytes, "the staged tile fits the LDS");
     __builtin_amdgcn_s_barrier();
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int i = 0; i < NA; ++i) {
+      const int nl = wn * 16 * NA + i * 16 + 4 * fq;
+      float b[4] = {0.0f, 0.0f, 0.0f, 0.0f}, c[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int i = 0; i < NA; ++i) {
-        const int nl = wn * 16 * NA + i * 16 + 4 * fq, ml = mw + j * kJS + fr;
-        float b[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (bias) {
+      for (int r = 0; r < 4; ++r) {
+        if (bias) b[r] = (n0 + nl + r < N) ? bias[n0 + nl + r] : 0.0f;
+        if (CH) c[r] = (n0 + nl + r < N) ? sw[n0 + nl + r] : 0.0f;
+      }
 #pragma unroll
-          for (int r = 0; r < 4; ++r) b[r] = (n0 + nl + r < N) ? bias[n0 + nl + r] : 0.0f;
+      for (int j = 0; j < 8; ++j) {
+        const int ml = mw + j * kJS + fr;
+        v4f v = acc[i][j];
+        if (CH) {
+          const float sam = sa[min(m0 + ml, M - 1)];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = fmaf(mul_rn(v[r], sam), c[r], b[r]);  // channel_out before its rounding
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] += b[r];
         }
-        const uint32_t h01 = bf16x2_rne(acc[i][j][0] + b[0], acc[i][j][1] + b[1]);
-        const uint32_t h23 = bf16x2_rne(acc[i][j][2] + b[2], acc[i][j][3] + b[3]);
-        *reinterpret_cast<uint2*>(smem + ml * kRS + nl * 2) = make_uint2(h01, h23);
+        *reinterpret_cast<uint2*>(smem + ml * kRS + nl * 2) = make_uint2(bf16x2_rne(v[0], v[1]), bf16x2_rne(v[2], v[3]));
       }
     }
     __syncthreads();
@@ -651,6 +641,26 @@ __device__ __forceinline__ void prefill256_body(int block, const uint8_t* __rest
 #pragma unroll
         for (int e = 0; e < 8; ++e)
           if (n + e < N) dst[e] = static_cast<uint16_t>(h[e >> 1] >> (16 * (e & 1)));
+      }
+    }
+    return;
+  }
+  if (CH) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j < jl) {
+        const int m = m0 + mw + j * kJS + fr;
+        if (m < M) {
+          const float sam = sa[m];
+          uint16_t* row = y + static_cast<int64_t>(m) * ldy;
+#pragma unroll
+          for (int i = 0; i < NA; ++i) {
+            const int n = n0 + wn * 16 * NA + i * 16 + 4 * fq;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (n + r < N) row[n + r] = channel_out(acc[i][j][r], sam, sw[n + r], bias ? bias[n + r] : 0.0f);
+          }
+        }
       }
     }
     return;
@@ -690,27 +700,27 @@ __global__ __launch_bounds__(512) void gemm_prefill256_kernel(const uint8_t* __r
 // n2 = N - wide columns).  One launch instead of two: workgroups of the second
 // range start on the CUs as the first range's finish, with no launch gap and
 // no idle tail between the ranges.
-template <bool HALF, bool WPACK>
+template <bool HALF, bool WPACK, bool CH = false>
 __global__ __launch_bounds__(512) void gemm_prefill256_split_kernel(
     int split, const uint8_t* __restrict__ qa, const float* __restrict__ sa, int64_t ldy, int M, int K, int G,
-    int Mpad, int gs, int64_t ldyp, int accum, const uint8_t* __restrict__ w1, const float* __restrict__ sw1,
+    int Mpad, int64_t ldq, int gs, int64_t ldyp, int accum, const uint8_t* __restrict__ w1, const float* __restrict__ sw1,
     const float* __restrict__ bias1, uint16_t* __restrict__ y1, float* __restrict__ yp1, int n1,
     const uint8_t* __restrict__ w2, const float* __restrict__ sw2, const float* __restrict__ bias2,
     uint16_t* __restrict__ y2, float* __restrict__ yp2, int n2) {
   const int b = static_cast<int>(blockIdx.x);
   if (b < split)
-    prefill256_body<HALF, false, false, WPACK, 4>(b, qa, sa, w1, sw1, bias1, y1, ldy, M, n1, K, G, Mpad, nullptr,
-                                                  nullptr, 0, 0, 0, 1, yp1, 0, gs, ldyp, accum, 0);
+    prefill256_body<HALF, false, CH, WPACK, 4>(b, qa, sa, w1, sw1, bias1, y1, ldy, M, n1, K, G, Mpad, nullptr,
+                                               nullptr, 0, 0, 0, 1, yp1, ldq, gs, ldyp, accum, 0);
   else
-    prefill256_body<HALF, false, false, WPACK, 3>(b - split, qa, sa, w2, sw2, bias2, y2, ldy, M, n2, K, G, Mpad,
-                                                  nullptr, nullptr, 0, 0, 0, 1, yp2, 0, gs, ldyp, accum, 0);
+    prefill256_body<HALF, false, CH, WPACK, 3>(b - split, qa, sa, w2, sw2, bias2, y2, ldy, M, n2, K, G, Mpad,
+                                               nullptr, nullptr, 0, 0, 0, 1, yp2, ldq, gs, ldyp, accum, 0);
 }
 
 // The 160 KB of dynamic LDS is above the default limit: raise it once per device.
 constexpr int kMaxDevices = 64;
 
-std::once_flag g_lds_once[kMaxDevices][40];
-hipError_t g_lds_err[kMaxDevices][40];
+std::once_flag g_lds_once[kMaxDevices][41];
+hipError_t g_lds_err[kMaxDevices][41];
 
 template <bool HALF, bool GROUPED, bool CH = false, bool WPACK = false, int NA = 4, bool SWI = false>
 hipError_t ensure_lds_limit() {
@@ -718,7 +728,7 @@ hipError_t ensure_lds_limit() {
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
-  // slots 32..35: the split kernel; 36..39: the fused SiLU-and-mul form (grouped, NA = 4)
+  // slots 32..35: the split kernel; 36..39: the fused SiLU-and-mul form (grouped, NA = 4); 40: the channel split
   constexpr int slot = SWI ? 36 + (HALF ? 1 : 0) + (WPACK ? 2 : 0)
                            : (HALF ? 1 : 0) + (GROUPED ? 2 : 0) + (CH ? 4 : 0) + (WPACK ? 8 : 0) + (NA == 3 ? 16 : 0);
   std::call_once(g_lds_once[dev][slot], [dev] {
@@ -729,32 +739,35 @@ hipError_t ensure_lds_limit() {
   return g_lds_err[dev][slot];
 }
 
-template <bool HALF, bool WPACK>
+template <bool HALF, bool WPACK, bool CH>
 hipError_t ensure_lds_limit_split() {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
-  constexpr int slot = 32 + (HALF ? 1 : 0) + (WPACK ? 2 : 0);
+  constexpr int slot = CH ? 40 : 32 + (HALF ? 1 : 0) + (WPACK ? 2 : 0);
   std::call_once(g_lds_once[dev][slot], [dev] {
-    g_lds_err[dev][slot] = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_prefill256_split_kernel<HALF, WPACK>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+    g_lds_err[dev][slot] =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_prefill256_split_kernel<HALF, WPACK, CH>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
   });
   return g_lds_err[dev][slot];
 }
 
-template <bool HALF, bool WPACK>
+template <bool HALF, bool WPACK, bool CH = false>
 hipError_t launch_split(const GemmArgs& a, int wide, hipStream_t stream) {
-  hipError_t e = ensure_lds_limit_split<HALF, WPACK>();
+  hipError_t e = ensure_lds_limit_split<HALF, WPACK, CH>();
   if (e != hipSuccess) return e;
   const int tiles_m = a.Mpad / kBM, n2 = a.N - wide;
   const int split = tiles_m * (wide / 256);
   const unsigned blocks = static_cast<unsigned>(split + tiles_m * ((n2 + 191) / 192));
   // Columns [wide, N): weight rows from `wide` (row-major: + wide * K bytes; packed:
   // 16-row tiles of gs * 2048 = K * 16 bytes, the same offset), scale rows from wide / 128.
-  gemm_prefill256_split_kernel<HALF, WPACK><<<blocks, 512, kLdsBytes, stream>>>(
-      split, a.qa, a.sa, a.ldy, a.M, a.K, a.G, a.Mpad, a.gstride(), a.ldyp, a.accumulate ? 1 : 0, a.w, a.sw, a.bias,
-      a.y, a.yp, wide, a.w + static_cast<int64_t>(wide) * a.K, a.sw + static_cast<int64_t>(wide / 128) * a.gstride(),
+  // (per-channel scales: one per column).
+  gemm_prefill256_split_kernel<HALF, WPACK, CH><<<blocks, 512, kLdsBytes, stream>>>(
+      split, a.qa, a.sa, a.ldy, a.M, a.K, a.G, a.Mpad, a.ldq, a.gstride(), a.ldyp, a.accumulate ? 1 : 0, a.w, a.sw,
+      a.bias, a.y, a.yp, wide, a.w + static_cast<int64_t>(wide) * a.K,
+      a.sw + (CH ? static_cast<int64_t>(wide) : static_cast<int64_t>(wide / 128) * a.gstride()),
       a.bias ? a.bias + wide : nullptr, a.y ? a.y + wide : nullptr, a.yp ? a.yp + wide : nullptr, n2);
   return hipGetLastError();
 }
@@ -807,10 +820,15 @@ hipError_t launch_gemm_channel256(const GemmArgs& a, hipStream_t stream) {
     return hipErrorInvalidValue;
   hipError_t e = ensure_lds_limit<false, false, true>();
   if (e != hipSuccess) return e;
-  const int mpad = (a.M + kBM - 1) / kBM * kBM;
-  const unsigned tiles = static_cast<unsigned>(((a.N + kBN - 1) / kBN) * (mpad / kBM));
+  GemmArgs c = a;
+  c.Mpad = (a.M + kBM - 1) / kBM * kBM;
+  const TileId tile = plan_tile(a.M, c.Mpad, a.N, device_cus());
+  if (tile != kTile256) return launch_gemm_tiles(c, tile, stream);
+  const int wide = prefill_wide_columns(c.Mpad, a.N, device_cus());
+  if (wide < a.N) return launch_split<false, false, true>(c, wide, stream);
+  const unsigned tiles = static_cast<unsigned>(((a.N + kBN - 1) / kBN) * (c.Mpad / kBM));
   gemm_prefill256_kernel<false, false, true><<<tiles, 512, kLdsBytes, stream>>>(
-      a.qa, a.sa, a.w, a.sw, a.bias, a.y, a.ldy, a.M, a.N, a.K, a.G, mpad, nullptr, nullptr, 0, 0, 0, 1, nullptr,
+      a.qa, a.sa, a.w, a.sw, a.bias, a.y, a.ldy, a.M, a.N, a.K, a.G, c.Mpad, nullptr, nullptr, 0, 0, 0, 1, nullptr,
       a.ldq, a.G, 0, 0, 0, nullptr, nullptr);
   return hipGetLastError();
 }

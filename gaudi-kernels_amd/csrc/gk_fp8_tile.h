@@ -67,6 +67,25 @@ __device__ inline uint16_t channel_out(float p, float sam, float swn, float bn) 
   return bf16_rne(fmaf(mul_rn(p, sam), swn, bn));
 }
 
+// The same on columns n .. n + 3 of token m (one 8-byte store where the row allows it).
+__device__ inline void store_channel_tile(uint16_t* __restrict__ y, int64_t ldy, const float* __restrict__ sw,
+                                          const float* __restrict__ bias, int N, int m, int n, float sam, v4f acc) {
+  uint16_t* row = y + static_cast<int64_t>(m) * ldy + n;
+  float v[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    v[r] = n + r < N ? fmaf(mul_rn(acc[r], sam), sw[n + r], bias ? bias[n + r] : 0.0f) : 0.0f;
+  const uint32_t h01 = bf16x2_rne(v[0], v[1]), h23 = bf16x2_rne(v[2], v[3]);
+  if (n + 3 < N && ((reinterpret_cast<uintptr_t>(row) & 7) == 0)) {
+    *reinterpret_cast<uint2*>(row) = make_uint2(h01, h23);
+  } else {
+    if (n < N) row[0] = static_cast<uint16_t>(h01);
+    if (n + 1 < N) row[1] = static_cast<uint16_t>(h01 >> 16);
+    if (n + 2 < N) row[2] = static_cast<uint16_t>(h23);
+    if (n + 3 < N) row[3] = static_cast<uint16_t>(h23 >> 16);
+  }
+}
+
 // Writes C[n0 + 4*quad + r][m] (r = 0..3) of one 16x16 tile as bf16 with bias.
 __device__ inline void store_tile(uint16_t* __restrict__ y, int64_t ldy, const float* __restrict__ bias, int M,
                                   int N, int m, int n, v4f acc) {

@@ -282,10 +282,7 @@ __device__ __forceinline__ void gemm_tile_body(
     for (int i = 0; i < NA; ++i) {
       const int n = nb + 16 * i;
       if (CH) {
-        uint16_t* row = y + static_cast<int64_t>(m) * ldy + n;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (n + r < N) row[r] = channel_out(acc[i][j][r], sam, sw[n + r], bias ? bias[n + r] : 0.0f);
+        store_channel_tile(y, ldy, sw, bias, N, m, n, sam, acc[i][j]);
       } else if (yp) {
         float* dst = yp + static_cast<int64_t>(m) * ldyp + n;
         if (n + 3 < N && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {

@@ -45,3 +45,27 @@ def test_tiles_equal_256_rows(m, n, k):
     w, s = synth.weight(n, k, seed=3, device="cuda")
     big = ops.block_fp8_gemm(x, w, s)
     assert torch.equal(ops.block_fp8_gemm(x[:m], w, s).view(torch.int16), big[:m].view(torch.int16))
+
+
+# 64x32, 64x64, 128x64, 128x64 twice a CU, 128x128, 256x256 in one range and (last) in two of 256 and 192 columns
+@pytest.mark.parametrize("m,n,k", [(17, 500, 384), (128, 6140, 640), (300, 6144, 256), (777, 5003, 384),
+                                   (1000, 4090, 128), (2047, 7168, 256), (4095, 7160, 256)])
+def test_channel_tiles(m, n, k):
+    """Every tile of the per-channel GEMM against 64-bit products: P is a sum of at most 640 exact products whose
+    fp8 matrix instruction sums to within 1e-4 of its scale; the rest is three fp32 roundings and the bf16 one."""
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    q, sa = ops.token_quant(torch.randn(m, k, generator=gen, device="cuda").bfloat16())
+    w = torch.randint(0, 127, (n, k), dtype=torch.uint8, device="cuda", generator=gen)
+    w |= torch.randint(0, 2, (n, k), dtype=torch.uint8, device="cuda", generator=gen) << 7
+    sw, bias = torch.rand(n, device="cuda", generator=gen), torch.randn(n, device="cuda", generator=gen)
+    out = torch.full((m + 1, n + 8), -1.0, dtype=torch.bfloat16, device="cuda")
+    ops.channel_gemm(q, sa, w, sw, bias, out=out[:m, :n])
+    assert bool((out[m] == -1).all()) and bool((out[:, n:] == -1).all())
+    a = q.view(torch.float8_e4m3fn).double()
+    p = (a @ w.view(torch.float8_e4m3fn).double().t()) * sa.double()[:, None] * sw.double()
+    scale = (a.abs() @ w.view(torch.float8_e4m3fn).double().abs().t()) * sa.double()[:, None] * sw.double()
+    err = (out[:m, :n].double() - (p + bias.double())).abs()
+    assert bool((err <= 2.0 ** -8 * (p + bias.double()).abs() + 1e-4 * scale + 1e-6).all())
+    odd = torch.empty(m, n + 1, dtype=torch.bfloat16, device="cuda")[:, :n]  # rows that take no wide stores
+    ops.channel_gemm(q, sa, w, sw, bias, out=odd)
+    assert torch.equal(odd.view(torch.int16), out[:m, :n].view(torch.int16))
