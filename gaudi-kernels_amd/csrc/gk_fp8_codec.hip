@@ -180,19 +180,20 @@ template <bool HALF, bool PACKED, int U>
 __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t* __restrict__ x, int64_t ldx, int M,
                                                         int K, int G, int Mpad, uint8_t* __restrict__ q,
                                                         float* __restrict__ sa, int vec_ok) {
-  const int64_t gid0 = (static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 4) + (threadIdx.x >> 4)) * U;
+  // 32-bit indices (a 64-bit division a group costs as much as the quantizer): the codes of 2^32 groups are 512 GB
+  const uint32_t gid0 = (blockIdx.x * (blockDim.x >> 4) + (threadIdx.x >> 4)) * U;
   const int sub = threadIdx.x & 15;
-  const int64_t total = static_cast<int64_t>(Mpad) * G;
+  const uint32_t total = static_cast<uint32_t>(Mpad) * static_cast<uint32_t>(G);
   uint4 raw[U];
   int64_t row[U];
   int gg[U];
   bool active[U], live[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int64_t gid = gid0 + u;
+    const uint32_t gid = gid0 + u, r = gid / static_cast<uint32_t>(G);
     active[u] = gid < total;
-    row[u] = active[u] ? gid / G : 0;
-    gg[u] = active[u] ? static_cast<int>(gid - row[u] * G) : 0;
+    row[u] = active[u] ? r : 0;
+    gg[u] = active[u] ? static_cast<int>(gid - r * static_cast<uint32_t>(G)) : 0;
     const int col = gg[u] * 128 + sub * 8;
     live[u] = active[u] && row[u] < M;
     raw[u] = make_uint4(0u, 0u, 0u, 0u);
@@ -208,7 +209,7 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t* __restri
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     float s;
-    const uint2 codes = quant_group8(raw[u], live[u], HALF, &s);  // all 16 lanes of a group take part
+    const uint2 codes = quant_group8(raw[u], true, HALF, &s);  // all 16 lanes of a group take part (zeros: not live)
     if (active[u]) {
       const int64_t slot = static_cast<int64_t>(gg[u]) * Mpad + row[u];
       // bytes [8 sub, 8 sub + 8): 16-byte chunk c = sub / 2 goes to piece (c % 2, 16 (c / 2) + row)

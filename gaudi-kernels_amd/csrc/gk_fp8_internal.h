@@ -38,9 +38,30 @@ __device__ inline uint32_t bf16x2_rne(float a, float b) {
 // both give the same bits.
 enum Act { kSilu = 0, kGeluErf = 1, kGeluTanh = 2 };
 
+// SiLU for |g| <= 80: the same quotient g / (1 + e^-g) without the range
+// handling of expf and of the IEEE division, which took most of the SiLU-and-mul
+// kernels' time (they are VALU-bound).  e^-g = 2^t with t = -g log2(e) in two
+// parts (the hardware exponential, 1 ulp, of the high part; the low one to first
+// order); the quotient is a refined reciprocal product whose residual keeps -0.
+// Every |g| <= 80 keeps e^-g, 1 + e^-g and the reciprocal normal and finite.
+// Within 2 ulps of the 64-bit value like silu_ref: the rounded products differ
+// from it in as few places (tests/test_gpu_silu_fast.py).
+__device__ inline float silu_fast(float g) {
+  const float hi = g * -1.44269502162933349609375f;  // fp32(-log2 e)
+  float lo = fmaf(g, -1.44269502162933349609375f, -hi);
+  lo = fmaf(g, -1.92596299112661746887e-8f, lo);  // log2 e - fp32(log2 e), negated
+  const float e0 = __builtin_amdgcn_exp2f(hi);
+  const float d = 1.0f + fmaf(e0, lo * 0.693147180559945f, e0);
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float q0 = g * r;
+  return fmaf(-fmaf(d, q0, -g), r, q0);
+}
+
+// One rule per element: silu_fast for |g| <= 80, silu_ref beyond (and NaN).
 template <int ACT>
 __device__ inline float act_ref(float g) {
-  return ACT == kSilu ? silu_ref(g) : ACT == kGeluErf ? gelu_erf_ref(g) : gelu_tanh_ref(g);
+  if (ACT == kSilu) return fabsf(g) <= 80.0f ? silu_fast(g) : silu_ref(g);
+  return ACT == kGeluErf ? gelu_erf_ref(g) : gelu_tanh_ref(g);
 }
 
 template <int ACT>
@@ -48,6 +69,34 @@ __device__ inline uint32_t act_mul_pair(uint32_t g2, uint32_t u2) {
   const float g0 = bits_f32(g2 << 16), g1 = bits_f32(g2 & 0xffff0000u);
   const float u0 = bits_f32(u2 << 16), u1 = bits_f32(u2 & 0xffff0000u);
   return bf16x2_rne(mul_rn(act_ref<ACT>(g0), u0), mul_rn(act_ref<ACT>(g1), u1));
+}
+
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+// The larger of the magnitudes (bits without the sign) in each half of four packed pairs.
+__device__ inline u16x2 mag_max4(uint4 v) {
+  auto m = [](uint32_t x) { return __builtin_bit_cast(u16x2, x & 0x7fff7fffu); };
+  return __builtin_elementwise_max(__builtin_elementwise_max(m(v.x), m(v.y)),
+                                   __builtin_elementwise_max(m(v.z), m(v.w)));
+}
+
+// act_mul_pair on eight values.  SiLU: when every gate is in silu_fast's range
+// and every up value finite (no product is NaN), without the special cases.
+template <int ACT>
+__device__ inline uint4 act_mul8(uint4 gv, uint4 uv) {
+  if (ACT == kSilu) {
+    const u16x2 g = mag_max4(gv), u = mag_max4(uv);
+    if (max(g[0], g[1]) <= 0x42a0 && max(u[0], u[1]) < 0x7f80) {  // bf16 80.0; infinity
+      auto two = [](uint32_t g2, uint32_t u2) {
+        const f32x2 v = {mul_rn(silu_fast(bits_f32(g2 << 16)), bits_f32(u2 << 16)),
+                         mul_rn(silu_fast(bits_f32(g2 & 0xffff0000u)), bits_f32(u2 & 0xffff0000u))};
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+      };
+      return make_uint4(two(gv.x, uv.x), two(gv.y, uv.y), two(gv.z, uv.z), two(gv.w, uv.w));
+    }
+  }
+  return make_uint4(act_mul_pair<ACT>(gv.x, uv.x), act_mul_pair<ACT>(gv.y, uv.y), act_mul_pair<ACT>(gv.z, uv.z),
+                    act_mul_pair<ACT>(gv.w, uv.w));
 }
 
 // Row padding of the quantized-activation workspace.

@@ -555,8 +555,7 @@ __device__ __forceinline__ void prefill256_body(int block, const uint8_t* __rest
       const uint32_t o = static_cast<uint32_t>(r * 256 + ((sub ^ (r & 15)) << 4));
       const uint4 gv = *reinterpret_cast<const uint4*>(smem + o);
       const uint4 uv = *reinterpret_cast<const uint4*>(smem + 65536 + o);
-      const uint4 h = make_uint4(act_mul_pair<kSilu>(gv.x, uv.x), act_mul_pair<kSilu>(gv.y, uv.y),
-                                 act_mul_pair<kSilu>(gv.z, uv.z), act_mul_pair<kSilu>(gv.w, uv.w));
+      const uint4 h = act_mul8<kSilu>(gv, uv);
       float s;
       const uint2 codes = quant_group8(h, true, HALF, &s);
       const int64_t slot = static_cast<int64_t>(tn) * Mpad + m0 + r;
