@@ -21,6 +21,8 @@ struct DecodeShape {
 #define GK_DECODE_SHAPES(X) GK_DECODE_SHAPES_T1(X)                                             \
   X(2, 2, 2, 2) X(2, 2, 1, 2) X(8, 2, 1, 2) X(8, 2, 2, 2) X(8, 1, 1, 2) X(16, 1, 1, 2)         \
   X(2, 2, 1, 4) X(8, 2, 1, 4) X(8, 1, 1, 4) X(16, 1, 1, 4)
+// The MT = 4 shapes computing three of the four tiles (M <= 48).
+#define GK_DECODE_SHAPES3(X) X(2, 2, 1, 3) X(8, 2, 1, 3) X(8, 1, 1, 3) X(16, 1, 1, 3)
 
 constexpr int decode_key(int nw, int r, int u, int mt) { return ((nw * 10 + r) * 10 + u) * 10 + mt; }
 
