@@ -336,15 +336,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_decode_kernel(const uint8_t* __r
 // instruction's own sums are coarser, 3e-5).  One 128-K group of a 16 x 16 block
 // is four of them; the group's sum takes its scales as in the other variants.
 //
-// Workgroup = kGW waves over 32 weight rows x 16 MB tokens, the groups dealt
-// round-robin to the waves; the kGW partial tiles are summed in wave order.  A
+// Workgroup = NW waves over 32 weight rows x 16 MB tokens, the groups dealt
+// round-robin to the waves; the NW partial tiles are summed in wave order.  A
 // wave stages its group in its own LDS (no barrier in the loop): 16-byte weight
 // loads at any byte alignment, or single bytes where a row's last chunk would
 // pass K (those past K become zero), the next group's loads in flight during the
 // current one's products.  Bound by the latency of a wave's few load rounds, so
 // the tile is small and K is split: M = 200, N = K = 2880 7.0 ms (byte loads, one
-// output a thread) -> 19.4 us.
-constexpr int kGW = 8;
+// output a thread) -> 15.7 us.
 
 // 8 E4M3 codes -> 8 bf16 values.
 __device__ inline bf16x8 widen8(uint32_t lo, uint32_t hi) {
@@ -355,8 +354,8 @@ __device__ inline bf16x8 widen8(uint32_t lo, uint32_t hi) {
   return bf16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
-template <int MB, bool HALF>
-__global__ __launch_bounds__(64 * kGW) void gemm_generic_kernel(const uint8_t* __restrict__ qa,
+template <int MB, int NW, bool HALF>
+__global__ __launch_bounds__(64 * NW) void gemm_generic_kernel(const uint8_t* __restrict__ qa,
                                                                 const float* __restrict__ sa,
                                                                 const uint8_t* __restrict__ w,
                                                                 const float* __restrict__ sw,
@@ -365,7 +364,7 @@ __global__ __launch_bounds__(64 * kGW) void gemm_generic_kernel(const uint8_t* _
                                                                 int K, int G, int Mpad, int tiles_m) {
   constexpr int NA = 2, kWaveLds = (16 * NA + 16 * MB) * 128;
   static_assert(kWaveLds >= NA * MB * 64 * 16, "the partial tile fits the wave's staging buffer");
-  __shared__ __attribute__((aligned(16))) uint8_t lds[kGW][kWaveLds];
+  __shared__ __attribute__((aligned(16))) uint8_t lds[NW][kWaveLds];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int n0 = static_cast<int>(blockIdx.x / tiles_m) * 16 * NA, m0 = static_cast<int>(blockIdx.x % tiles_m) * 16 * MB;
@@ -411,7 +410,7 @@ __global__ __launch_bounds__(64 * kGW) void gemm_generic_kernel(const uint8_t* _
 #pragma unroll
     for (int j = 0; j < MB; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   if (wave < G) load(wave);
-  for (int g = wave; g < G; g += kGW) {
+  for (int g = wave; g < G; g += NW) {
     float f[MB];
 #pragma unroll
     for (int j = 0; j < MB; ++j) {
@@ -430,7 +429,7 @@ __global__ __launch_bounds__(64 * kGW) void gemm_generic_kernel(const uint8_t* _
       const int r = 8 * i + lr;
       *reinterpret_cast<u32x4*>(al + r * 128 + ((lc ^ lds_key(r)) << 4)) = ar[i];
     }
-    if (g + kGW < G) load(g + kGW);
+    if (g + NW < G) load(g + NW);
     // fragments: lane -> row lane % 16, K bytes [32 (lane / 16), +32); product s takes bytes [8 s, 8 s + 8) of
     // those on both sides, so together the four cover the group once
     bf16x8 b[MB][4];
@@ -461,11 +460,11 @@ __global__ __launch_bounds__(64 * kGW) void gemm_generic_kernel(const uint8_t* _
 #pragma unroll
     for (int j = 0; j < MB; ++j) *reinterpret_cast<v4f*>(wl + (i * MB + j) * 1024 + lane * 16) = acc[i][j];
   __syncthreads();
-  // wave t sums block t of the kGW partial tiles in wave order
-  for (int t = wave; t < NA * MB; t += kGW) {
+  // wave t sums block t of the NW partial tiles in wave order
+  for (int t = wave; t < NA * MB; t += NW) {
     v4f sum = *reinterpret_cast<const v4f*>(lds[0] + t * 1024 + lane * 16);
 #pragma unroll
-    for (int v = 1; v < kGW; ++v) sum += *reinterpret_cast<const v4f*>(lds[v] + t * 1024 + lane * 16);
+    for (int v = 1; v < NW; ++v) sum += *reinterpret_cast<const v4f*>(lds[v] + t * 1024 + lane * 16);
     store_tile(y, ldy, bias, M, N, m0 + 16 * (t % MB) + fr, n0 + 16 * (t / MB) + 4 * fq, sum);
   }
 }
@@ -564,22 +563,26 @@ hipError_t launch_gemm_token_channel(const GemmArgs& a, hipStream_t stream) {
   }
 }
 
-template <int MB>
-static hipError_t generic_launch(const GemmArgs& a, hipStream_t stream) {
-  const int64_t tiles_m = (a.M + 16 * MB - 1LL) / (16 * MB), tiles = tiles_m * ((a.N + 31LL) / 32);
+template <int MB, int NW>
+static hipError_t generic_launch(const GemmArgs& a, int64_t tiles_m, int64_t tiles, hipStream_t stream) {
   if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
   if (a.half_w)
-    gemm_generic_kernel<MB, true><<<static_cast<unsigned>(tiles), 64 * kGW, 0, stream>>>(
+    gemm_generic_kernel<MB, NW, true><<<static_cast<unsigned>(tiles), 64 * NW, 0, stream>>>(
         a.qa, a.sa, a.w, a.sw, a.bias, a.y, a.ldy, a.M, a.N, a.K, a.G, a.Mpad, static_cast<int>(tiles_m));
   else
-    gemm_generic_kernel<MB, false><<<static_cast<unsigned>(tiles), 64 * kGW, 0, stream>>>(
+    gemm_generic_kernel<MB, NW, false><<<static_cast<unsigned>(tiles), 64 * NW, 0, stream>>>(
         a.qa, a.sa, a.w, a.sw, a.bias, a.y, a.ldy, a.M, a.N, a.K, a.G, a.Mpad, static_cast<int>(tiles_m));
   return hipGetLastError();
 }
 
 hipError_t launch_gemm_generic(const GemmArgs& a, hipStream_t stream) {
-  // up to 16 tokens fill one block; beyond, two share each weight fragment
-  return a.M <= 16 ? generic_launch<1>(a, stream) : generic_launch<2>(a, stream);
+  // Up to 16 tokens fill one block; beyond, two share each weight fragment.  Eight waves split K while a CU has one
+  // workgroup anyway; with more workgroups than CUs four (three workgroups a CU by registers instead of one: M = 200,
+  // N = K = 2880 19.4 -> 15.7 us; M = 20 there, 90 workgroups: 7.4 us with four waves, 6.4 with eight).
+  const int64_t tiles_n = (a.N + 31LL) / 32;
+  if (a.M <= 16) return generic_launch<1, 8>(a, 1, tiles_n, stream);
+  const int64_t tiles_m = (a.M + 31LL) / 32, tiles = tiles_m * tiles_n;
+  return tiles <= 256 ? generic_launch<2, 8>(a, tiles_m, tiles, stream) : generic_launch<2, 4>(a, tiles_m, tiles, stream);
 }
 
 }  // namespace gk
