@@ -4,14 +4,16 @@
 // and both fused with the 1x128 activation quantizer (codes + scales ready
 // for the block-FP8 GEMM that consumes the normalized rows).
 //
-// Per row (one workgroup of 256 threads; thread t holds the 8-element chunks
-// t, t + 256, ... in registers, at most four for width <= 8192):
+// Per row (one workgroup of NT = 256, 512 or 1024 threads; thread t holds the
+// 8-element chunks t, t + NT, ... in registers, at most four for width <= 8192):
 //   add        r = bf16_rne(fp32(x) + fp32(residual))  (fused form; residual_out = r)
 //   sum        ss = fp32 of the fp64 sum of r*r: each square is exact in
 //              fp64; thread t adds its chunks' squares in element order; each
 //              wave folds its 64 partial sums pairwise (lane l += lane l + s,
-//              s = 32 .. 1, by butterfly shuffles), and the four wave sums are
-//              folded the same way (s = 2, 1).
+//              s = 32 .. 1, by butterfly shuffles), and the wave sums are
+//              folded the same way.  (Sums of bf16 squares whose magnitudes
+//              lie within 2^12 of each other are exact in fp64, so NT does
+//              not change them.)
 //   inverse    inv = fp32(1 / sqrt(fp64(ss * fp32(1/width) + eps))), the
 //              multiply and the add in fp32 as the reference's expression
 //              (rms_norm_bf16.c:24-25), then an fp64 square root and division
@@ -20,7 +22,7 @@
 // The reference joins fp32 lane sums with a compensated reduction and
 // refines a hardware rsqrt (norm_math.h:5-23); both target the correctly
 // rounded values that the fp64 steps here give.  The CPU restatement
-// (oracle/norm.py) follows the same order, so the outputs are compared bit
+// (oracle/norm.py) follows the order of NT = 256, so the outputs are compared bit
 // for bit, and against the reference test's own gate (2 bf16 ulps of an
 // fp64 evaluation, tests/track_a_device_verify.cpp:490-540).
 //
@@ -37,8 +39,7 @@ namespace gk {
 
 namespace {
 
-constexpr int kNormThreads = 256;
-constexpr int kNormPasses = kNormMaxWidth / (8 * kNormThreads);  // 4
+constexpr int kNormThreads = 256;  // many rows; few rows take more threads a row (launch_rms_norm)
 
 __device__ inline float lo_bf16(uint32_t w) { return bits_f32(w << 16); }
 __device__ inline float hi_bf16(uint32_t w) { return bits_f32(w & 0xffff0000u); }
@@ -75,21 +76,21 @@ __device__ inline uint32_t norm_pair(uint32_t v, uint32_t g, float inv, float of
   return bf16x2_rne(n0, n1);
 }
 
-template <bool ADD, bool QUANT, bool HALF, bool PACKED, bool VEC>
-__global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(
+template <int NT, int PASSES, bool ADD, bool QUANT, bool HALF, bool PACKED, bool VEC>
+__global__ __launch_bounds__(NT) void rms_norm_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ res, int64_t ld_in, const uint16_t* __restrict__ gamma,
     int rows, int width, float eps, float off, uint16_t* __restrict__ res_out, uint16_t* __restrict__ norm_out,
     int64_t ld_out, uint8_t* __restrict__ q, float* __restrict__ sa, int Mpad) {
-  __shared__ double wsum[kNormThreads / 64];
+  __shared__ double wsum[NT / 64];
   const int t = threadIdx.x;
   const int row = blockIdx.x;
   const int G = (width + 127) >> 7;
   const bool live = row < rows;  // QUANT grids cover Mpad rows; rows past `rows` write zeros
-  uint4 v[kNormPasses], gv[kNormPasses];
+  uint4 v[PASSES], gv[PASSES];
   double acc = 0.0;
 #pragma unroll
-  for (int p = 0; p < kNormPasses; ++p) {
-    const int c = 8 * (t + kNormThreads * p);
+  for (int p = 0; p < PASSES; ++p) {
+    const int c = 8 * (t + NT * p);
     v[p] = make_uint4(0u, 0u, 0u, 0u);
     gv[p] = make_uint4(0u, 0u, 0u, 0u);
     if (live && c < width) {
@@ -119,13 +120,20 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(
   for (int s = 32; s >= 1; s >>= 1) acc = acc + __shfl_xor(acc, s, 64);
   if ((t & 63) == 0) wsum[t >> 6] = acc;
   __syncthreads();
-  const float ss = static_cast<float>((wsum[0] + wsum[2]) + (wsum[1] + wsum[3]));
+  double w[NT / 64];  // the wave sums folded pairwise (s = NT / 128 .. 1), by every thread
+#pragma unroll
+  for (int i = 0; i < NT / 64; ++i) w[i] = wsum[i];
+#pragma unroll
+  for (int s = NT / 128; s >= 1; s >>= 1)
+#pragma unroll
+    for (int i = 0; i < s; ++i) w[i] = w[i] + w[i + s];
+  const float ss = static_cast<float>(w[0]);
   const float arg = add_rn(mul_rn(ss, 1.0f / static_cast<float>(width)), eps);
   const float inv = arg == __builtin_inff() ? 0.0f : static_cast<float>(1.0 / sqrt(static_cast<double>(arg)));
 
 #pragma unroll
-  for (int p = 0; p < kNormPasses; ++p) {
-    const int chunk = t + kNormThreads * p;
+  for (int p = 0; p < PASSES; ++p) {
+    const int chunk = t + NT * p;
     const int c = 8 * chunk;
     uint4 n = make_uint4(0u, 0u, 0u, 0u);
     if (live && c < width) {
@@ -142,7 +150,7 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(
         n = make_uint4(w[0], w[1], w[2], w[3]);
       }
     }
-    if (QUANT && 8 * kNormThreads * p < width) {
+    if (QUANT && 8 * NT * p < width) {
       // The 16 lanes of this DPP row hold one 128-column group; groups past
       // the last are not stored.  quant_group8 runs on every lane of the
       // workgroup (the condition is uniform).
@@ -171,9 +179,20 @@ hipError_t launch_rms_norm(const uint16_t* x, const uint16_t* res, int64_t ld_in
   const bool vec = al16(x) && (!res || al16(res)) && al16(gamma) && (!res_out || al16(res_out)) &&
                    (!norm_out || al16(norm_out)) && ld_in % 8 == 0 && ld_out % 8 == 0;
   const unsigned grid = static_cast<unsigned>(quant ? Mpad : rows);
-#define GK_NORM(A, Q, H, P, V)                                                                             \
-  rms_norm_kernel<A, Q, H, P, V><<<grid, kNormThreads, 0, stream>>>(x, res, ld_in, gamma, rows, width, eps, off, \
-                                                                     res_out, norm_out, ld_out, q, sa, Mpad)
+  // A row's work is a chain of a few hundred instructions a pass (fp64 sums, then the quantizer), about 0.7 us, which
+  // nothing hides while there are at most as many rows as CUs: then a row takes one pass, with 512 or 1024 threads
+  // beyond 2048 columns.  More rows hide it themselves and keep 256 threads (16 x 4096 with residual and quantizer:
+  // 4.2 -> 3.7 us, 16 x 7168 5.8 -> 4.6; 4093 x 4096 24.4 us either way).
+  const int nt = grid > 256 || width <= 8 * 256 ? 256 : width <= 8 * 512 ? 512 : 1024;
+#define GK_NORM_T(NT, PASSES, A, Q, H, P, V)                                                               \
+  rms_norm_kernel<NT, PASSES, A, Q, H, P, V><<<grid, NT, 0, stream>>>(x, res, ld_in, gamma, rows, width, eps, off, \
+                                                                      res_out, norm_out, ld_out, q, sa, Mpad)
+#define GK_NORM(A, Q, H, P, V)                              \
+  do {                                                      \
+    if (nt == 1024) GK_NORM_T(1024, 1, A, Q, H, P, V);      \
+    else if (nt == 512) GK_NORM_T(512, 1, A, Q, H, P, V);   \
+    else GK_NORM_T(256, 4, A, Q, H, P, V);                  \
+  } while (0)
 #define GK_NORM_V(A, Q, H, P) \
   if (vec) GK_NORM(A, Q, H, P, true); else GK_NORM(A, Q, H, P, false)
 #define GK_NORM_Q(A)                                       \
@@ -188,6 +207,7 @@ hipError_t launch_rms_norm(const uint16_t* x, const uint16_t* res, int64_t ld_in
 #undef GK_NORM_Q
 #undef GK_NORM_V
 #undef GK_NORM
+#undef GK_NORM_T
   return hipGetLastError();
 }
 
