@@ -112,8 +112,14 @@ Status* take_slot() {
   if (!g_slots_tried) {
     g_slots_tried = true;
     void* p = nullptr;
+    // relaxed: the allocation must not end a capture that another thread has under way
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (hipHostMalloc(&p, kStatusSlots * sizeof(Status), hipHostMallocPortable | hipHostMallocMapped) == hipSuccess)
       g_slots = static_cast<Status*>(p);
+    else
+      (void)hipGetLastError();  // this call copies instead: the next launch check must not find the error
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
   }
   if (!g_slots || g_slots_used == ~uint64_t{0}) return nullptr;
   const int i = __builtin_ctzll(~g_slots_used);

@@ -39,8 +39,6 @@ namespace gk {
 
 namespace {
 
-constexpr int kNormThreads = 256;  // many rows; few rows take more threads a row (launch_rms_norm)
-
 __device__ inline float lo_bf16(uint32_t w) { return bits_f32(w << 16); }
 __device__ inline float hi_bf16(uint32_t w) { return bits_f32(w & 0xffff0000u); }
 
