@@ -595,7 +595,7 @@ __device__ __forceinline__ void prefill256_body(int block, const uint8_t* __rest
     // layout would store 32-byte pieces of 16 rows per instruction; every
     // workgroup of a round stores its tile at once, so the epilogue is a
     // write burst (measured on MI355X, config 4 GEMM: -1%; the channel form,
-    // which stored single values: M = 2048, N = 7168, K = 4096 101 -> 68 us).
+    // which stored single values: M = 2048, N = 7168, K = 4096 105 -> 60 us a call).
     // Same bits as store_tile and channel_out: fp32, one bf16 rounding.
     constexpr int kRS = BN * 2 + 16, kCPR = BN / 8;  // LDS row stride; 16-byte chunks per row
     static_assert(kBM * kRS <= kLdsBytes, "the staged tile fits the LDS");
