@@ -336,14 +336,17 @@ __global__ __launch_bounds__(NW * 64) void gemm_decode_kernel(const uint8_t* __r
 // instruction's own sums are coarser, 3e-5).  One 128-K group of a 16 x 16 block
 // is four of them; the group's sum takes its scales as in the other variants.
 //
-// Workgroup = NW waves over 32 weight rows x 16 MB tokens, the groups dealt
-// round-robin to the waves; the NW partial tiles are summed in wave order.  A
-// wave stages its group in its own LDS (no barrier in the loop): 16-byte weight
-// loads at any byte alignment, or single bytes where a row's last chunk would
-// pass K (those past K become zero), the next group's loads in flight during the
-// current one's products.  Bound by the latency of a wave's few load rounds, so
-// the tile is small and K is split: M = 200, N = K = 2880 7.0 ms (byte loads, one
-// output a thread) -> 15.7 us.
+// Workgroup = NW waves over 32 weight rows x 16 MB tokens.  Group g belongs to
+// partial sum g % 8, and the eight partial tiles are summed in that order,
+// whatever NW: a wave of four computes two of them one after the other, so a
+// token's bits depend on neither the batch nor the number of workgroups (which
+// costs 0.4 us of the time below).  A wave stages its group in
+// its own LDS (no barrier in the loop): 16-byte weight loads at any byte
+// alignment, or single bytes where a row's last chunk would pass K (those past K
+// become zero), the next group's loads in flight during the current one's
+// products.  Bound by the latency of a wave's few load rounds, so the tile is
+// small and K is split: M = 200, N = K = 2880 7.0 ms (byte loads, one output a
+// thread) -> 15.4 us.
 
 // 8 E4M3 codes -> 8 bf16 values.
 __device__ inline bf16x8 widen8(uint32_t lo, uint32_t hi) {
@@ -354,16 +357,17 @@ __device__ inline bf16x8 widen8(uint32_t lo, uint32_t hi) {
   return bf16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
+// Three waves a SIMD: registers for three workgroups of four waves a CU, the second partial sum included.
 template <int MB, int NW, bool HALF>
-__global__ __launch_bounds__(64 * NW) void gemm_generic_kernel(const uint8_t* __restrict__ qa,
+__global__ __launch_bounds__(64 * NW, 3) void gemm_generic_kernel(const uint8_t* __restrict__ qa,
                                                                 const float* __restrict__ sa,
                                                                 const uint8_t* __restrict__ w,
                                                                 const float* __restrict__ sw,
                                                                 const float* __restrict__ bias,
                                                                 uint16_t* __restrict__ y, int64_t ldy, int M, int N,
                                                                 int K, int G, int Mpad, int tiles_m) {
-  constexpr int NA = 2, kWaveLds = (16 * NA + 16 * MB) * 128;
-  static_assert(kWaveLds >= NA * MB * 64 * 16, "the partial tile fits the wave's staging buffer");
+  constexpr int NA = 2, P = 8 / NW, kWaveLds = (16 * NA + 16 * MB) * 128;  // P partial sums a wave
+  static_assert(kWaveLds >= P * NA * MB * 64 * 16, "the partial tiles fit the wave's staging buffer");
   __shared__ __attribute__((aligned(16))) uint8_t lds[NW][kWaveLds];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -404,13 +408,17 @@ __global__ __launch_bounds__(64 * NW) void gemm_generic_kernel(const uint8_t* __
   const float* sap[MB];
 #pragma unroll
   for (int j = 0; j < MB; ++j) sap[j] = sa + min(m0 + 16 * j + fr, M - 1);
-  v4f acc[NA][MB];
+  v4f acc[NA][MB], first[NA][MB];
 #pragma unroll
   for (int i = 0; i < NA; ++i)
 #pragma unroll
-    for (int j = 0; j < MB; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < MB; ++j) acc[i][j] = first[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   if (wave < G) load(wave);
-  for (int g = wave; g < G; g += NW) {
+  bool second = false;  // this wave's second partial sum is under way
+  for (int g = wave; g < G;) {
+    int next = g + 8;  // the wave's next group
+    const bool change = P > 1 && !second && next >= G && wave + NW < G;
+    if (change) next = wave + NW;
     float f[MB];
 #pragma unroll
     for (int j = 0; j < MB; ++j) {
@@ -429,7 +437,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_generic_kernel(const uint8_t* __
       const int r = 8 * i + lr;
       *reinterpret_cast<u32x4*>(al + r * 128 + ((lc ^ lds_key(r)) << 4)) = ar[i];
     }
-    if (g + NW < G) load(g + NW);
+    if (next < G) load(next);
     // fragments: lane -> row lane % 16, K bytes [32 (lane / 16), +32); product s takes bytes [8 s, 8 s + 8) of
     // those on both sides, so together the four cover the group once
     bf16x8 b[MB][4];
@@ -454,17 +462,33 @@ __global__ __launch_bounds__(64 * NW) void gemm_generic_kernel(const uint8_t* __
         for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaf(t[r], f[j], acc[i][j][r]);
       }
     }
+    if (change) {
+      second = true;
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+#pragma unroll
+        for (int j = 0; j < MB; ++j) {
+          first[i][j] = acc[i][j];
+          acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+    g = next;
   }
 #pragma unroll
-  for (int i = 0; i < NA; ++i)
+  for (int p = 0; p < P; ++p)
 #pragma unroll
-    for (int j = 0; j < MB; ++j) *reinterpret_cast<v4f*>(wl + (i * MB + j) * 1024 + lane * 16) = acc[i][j];
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int j = 0; j < MB; ++j)
+        *reinterpret_cast<v4f*>(wl + ((p * NA + i) * MB + j) * 1024 + lane * 16) =
+            p == (second ? 1 : 0) ? acc[i][j] : first[i][j];
   __syncthreads();
-  // wave t sums block t of the NW partial tiles in wave order
+  // wave t sums block t of the eight partial tiles (v of wave v % NW) in order
   for (int t = wave; t < NA * MB; t += NW) {
     v4f sum = *reinterpret_cast<const v4f*>(lds[0] + t * 1024 + lane * 16);
 #pragma unroll
-    for (int v = 1; v < NW; ++v) sum += *reinterpret_cast<const v4f*>(lds[v] + t * 1024 + lane * 16);
+    for (int v = 1; v < 8; ++v)
+      sum += *reinterpret_cast<const v4f*>(lds[v % NW] + (v / NW * NA * MB + t) * 1024 + lane * 16);
     store_tile(y, ldy, bias, M, N, m0 + 16 * (t % MB) + fr, n0 + 16 * (t / MB) + 4 * fq, sum);
   }
 }
@@ -578,7 +602,7 @@ static hipError_t generic_launch(const GemmArgs& a, int64_t tiles_m, int64_t til
 hipError_t launch_gemm_generic(const GemmArgs& a, hipStream_t stream) {
   // Up to 16 tokens fill one block; beyond, two share each weight fragment.  Eight waves split K while a CU has one
   // workgroup anyway; with more workgroups than CUs four (three workgroups a CU by registers instead of one: M = 200,
-  // N = K = 2880 19.4 -> 15.7 us; M = 20 there, 90 workgroups: 7.4 us with four waves, 6.4 with eight).
+  // N = K = 2880 19.4 -> 15.4 us; M = 20 there, 90 workgroups: 7.4 us with four waves, 6.4 with eight).
   const int64_t tiles_n = (a.N + 31LL) / 32;
   if (a.M <= 16) return generic_launch<1, 8>(a, 1, tiles_n, stream);
   const int64_t tiles_m = (a.M + 31LL) / 32, tiles = tiles_m * tiles_n;

@@ -36,3 +36,16 @@ def test_generic_edges(m, n, k, half, offset):
     assert max_rel <= block_fp8.MAX_REL_TOL and mean_rel <= block_fp8.MEAN_REL_TOL
     want = ref.to(torch.bfloat16) if ref.dtype != torch.bfloat16 else ref
     assert float((y != want).float().mean()) <= 0.01 or y.numel() < 100
+
+
+@pytest.mark.parametrize("n,k", [(2880, 2850), (200, 1000)])
+@pytest.mark.parametrize("half", [False, True])
+def test_generic_rows_do_not_depend_on_the_batch(n, k, half):
+    """A token's bits are the same alone, in one block of tokens and at either count of waves a workgroup (N = 2880:
+    M = 64 has 180 workgroups, M = 200 has 630)."""
+    x = synth.activations(200, k, seed=7).cuda()
+    w, s = synth.weight(n, k, seed=8)
+    w, s = w.cuda(), s.cuda()
+    big = ops.block_fp8_gemm(x, w, s, native_half=half).view(torch.int16)
+    for m in (1, 17, 64):
+        assert torch.equal(ops.block_fp8_gemm(x[:m], w, s, native_half=half).view(torch.int16), big[:m])
