@@ -432,6 +432,15 @@ __global__ __launch_bounds__(64 * NW, 3) void gemm_generic_kernel(const uint8_t*
       const int r = 8 * i + lr;
       *reinterpret_cast<u32x4*>(wl + r * 128 + ((lc ^ lds_key(r)) << 4)) = v;
     }
+    if (g * 128 + 128 > K) {  // codes past K do not count: a NaN code there times the weights' zeros would be NaN
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int bytes = K - (g * 128 + 16 * lc + 4 * e);
+        const uint32_t keep = bytes >= 4 ? ~0u : bytes > 0 ? ~0u >> (8 * (4 - bytes)) : 0u;
+#pragma unroll
+        for (int i = 0; i < 2 * MB; ++i) ar[i][e] &= keep;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < 2 * MB; ++i) {
       const int r = 8 * i + lr;

@@ -49,3 +49,14 @@ def test_generic_rows_do_not_depend_on_the_batch(n, k, half):
     big = ops.block_fp8_gemm(x, w, s, native_half=half).view(torch.int16)
     for m in (1, 17, 64):
         assert torch.equal(ops.block_fp8_gemm(x[:m], w, s, native_half=half).view(torch.int16), big[:m])
+
+
+@pytest.mark.parametrize("m", [5, 40])
+def test_generic_reads_no_codes_past_k(m):
+    """The codes of the last group's columns past K may hold anything, NaN codes included."""
+    n, k = 70, 1000
+    w, s = synth.weight(n, k, seed=1)
+    q, sa = ops.act_quant(synth.activations(m, k, seed=2).cuda())
+    y = ops.block_fp8_gemm_q(q, sa, m, w.cuda(), s.cuda())
+    q[-1, :, k % 128:] = 0x7F
+    assert torch.equal(ops.block_fp8_gemm_q(q, sa, m, w.cuda(), s.cuda()).view(torch.int16), y.view(torch.int16))
