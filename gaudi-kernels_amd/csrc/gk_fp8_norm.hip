@@ -11,9 +11,10 @@
 //              fp64; thread t adds its chunks' squares in element order; each
 //              wave folds its 64 partial sums pairwise (lane l += lane l + s,
 //              s = 32 .. 1, by butterfly shuffles), and the wave sums are
-//              folded the same way.  (Sums of bf16 squares whose magnitudes
-//              lie within 2^12 of each other are exact in fp64, so NT does
-//              not change them.)
+//              folded the same way.  The order of NT = 256 defines the result:
+//              more threads add in another one, and where that could round ss
+//              another way (order_matters) the row is summed again in it, so a
+//              row's bits do not depend on the number of rows.
 //   inverse    inv = fp32(1 / sqrt(fp64(ss * fp32(1/width) + eps))), the
 //              multiply and the add in fp32 as the reference's expression
 //              (rms_norm_bf16.c:24-25), then an fp64 square root and division
@@ -22,8 +23,8 @@
 // The reference joins fp32 lane sums with a compensated reduction and
 // refines a hardware rsqrt (norm_math.h:5-23); both target the correctly
 // rounded values that the fp64 steps here give.  The CPU restatement
-// (oracle/norm.py) follows the order of NT = 256, so the outputs are compared bit
-// for bit, and against the reference test's own gate (2 bf16 ulps of an
+// (oracle/norm.py) follows the order of NT = 256, so the outputs are compared
+// bit for bit, and against the reference test's own gate (2 bf16 ulps of an
 // fp64 evaluation, tests/track_a_device_verify.cpp:490-540).
 //
 // QUANT: the normalized bf16 values are quantized per 1x128 group by
@@ -74,6 +75,46 @@ __device__ inline uint32_t norm_pair(uint32_t v, uint32_t g, float inv, float of
   return bf16x2_rne(n0, n1);
 }
 
+// acc plus the squares of eight values, element 0, 1, ..., 7 (a bf16 square is
+// exact in fp64, so a contracted fma gives the same sums).
+__device__ inline double add_squares(double acc, uint4 a) {
+  const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    acc += static_cast<double>(lo_bf16(w[i])) * lo_bf16(w[i]);
+    acc += static_cast<double>(hi_bf16(w[i])) * hi_bf16(w[i]);
+  }
+  return acc;
+}
+
+// Wave sums of squares in wsum[64-thread wave] (lane l takes acc(l) + acc(l ^ s):
+// on lane 0 this is the pairwise fold).
+__device__ inline void wave_sum(double acc, int t, double* wsum) {
+#pragma unroll
+  for (int s = 32; s >= 1; s >>= 1) acc = acc + __shfl_xor(acc, s, 64);
+  if ((t & 63) == 0) wsum[t >> 6] = acc;
+}
+
+// The wave sums folded pairwise (s = NW / 2 .. 1), by every thread.
+template <int NW>
+__device__ inline double fold_waves(const double* wsum) {
+  double w[NW];
+#pragma unroll
+  for (int i = 0; i < NW; ++i) w[i] = wsum[i];
+#pragma unroll
+  for (int s = NW / 2; s >= 1; s >>= 1)
+#pragma unroll
+    for (int i = 0; i < s; ++i) w[i] = w[i] + w[i + s];
+  return w[0];
+}
+
+// Whether another order of the same sum could round to another fp32 value.  A sum of nonnegative terms is within
+// d * 2^-53 of the exact one (relative), d the additions on its longest path: 40 with 256 threads, 18 with more, so
+// the two lie within 2^-47 of each other.  True for a NaN.
+__device__ inline bool order_matters(double sum) {
+  return !(static_cast<float>(sum * (1.0 - 0x1p-46)) == static_cast<float>(sum * (1.0 + 0x1p-46)));
+}
+
 template <int NT, int PASSES, bool ADD, bool QUANT, bool HALF, bool PACKED, bool VEC>
 __global__ __launch_bounds__(NT) void rms_norm_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ res, int64_t ld_in, const uint16_t* __restrict__ gamma,
@@ -101,31 +142,29 @@ __global__ __launch_bounds__(NT) void rms_norm_kernel(
         if (res_out) store8<VEC>(res_out + static_cast<int64_t>(row) * ld_out, c, width, a);
       }
       v[p] = a;
-      // element order within the chunk: 0, 1, ..., 7 (a bf16 square is exact
-      // in fp64, so a contracted fma gives the same sums)
-      acc += static_cast<double>(lo_bf16(a.x)) * lo_bf16(a.x);
-      acc += static_cast<double>(hi_bf16(a.x)) * hi_bf16(a.x);
-      acc += static_cast<double>(lo_bf16(a.y)) * lo_bf16(a.y);
-      acc += static_cast<double>(hi_bf16(a.y)) * hi_bf16(a.y);
-      acc += static_cast<double>(lo_bf16(a.z)) * lo_bf16(a.z);
-      acc += static_cast<double>(hi_bf16(a.z)) * hi_bf16(a.z);
-      acc += static_cast<double>(lo_bf16(a.w)) * lo_bf16(a.w);
-      acc += static_cast<double>(hi_bf16(a.w)) * hi_bf16(a.w);
+      acc = add_squares(acc, a);
     }
   }
-  // lane l takes acc(l) + acc(l ^ s): on lane 0 this is the pairwise fold
-#pragma unroll
-  for (int s = 32; s >= 1; s >>= 1) acc = acc + __shfl_xor(acc, s, 64);
-  if ((t & 63) == 0) wsum[t >> 6] = acc;
+  wave_sum(acc, t, wsum);
   __syncthreads();
-  double w[NT / 64];  // the wave sums folded pairwise (s = NT / 128 .. 1), by every thread
+  double sum = fold_waves<NT / 64>(wsum);
+  if constexpr (NT > 256) {
+    static_assert(PASSES == 1, "a row's chunks are all in v[0]");
+    if (order_matters(sum)) {  // every thread has the same sum
+      __shared__ uint4 chunks[NT];
+      chunks[t] = v[0];
+      __syncthreads();  // every thread has read wsum, too
+      double again = 0.0;
+      if (t < 256) {
 #pragma unroll
-  for (int i = 0; i < NT / 64; ++i) w[i] = wsum[i];
-#pragma unroll
-  for (int s = NT / 128; s >= 1; s >>= 1)
-#pragma unroll
-    for (int i = 0; i < s; ++i) w[i] = w[i] + w[i + s];
-  const float ss = static_cast<float>(w[0]);
+        for (int p = 0; p < NT / 256; ++p) again = add_squares(again, chunks[t + 256 * p]);
+        wave_sum(again, t, wsum);
+      }
+      __syncthreads();
+      sum = fold_waves<4>(wsum);
+    }
+  }
+  const float ss = static_cast<float>(sum);
   const float arg = add_rn(mul_rn(ss, 1.0f / static_cast<float>(width)), eps);
   const float inv = arg == __builtin_inff() ? 0.0f : static_cast<float>(1.0 / sqrt(static_cast<double>(arg)));
 
