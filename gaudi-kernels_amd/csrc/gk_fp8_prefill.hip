@@ -840,7 +840,9 @@ hipError_t launch_gemm_channel256(const GemmArgs& a, hipStream_t stream) {
 // per-element arithmetic.
 hipError_t launch_gemm_prefill256(const GemmArgs& a, hipStream_t stream) {
   if (a.Mpad % kBM != 0 || !prefill256_fits(a)) return hipErrorInvalidValue;
-  const TileId tile = plan_tile(a.M, a.Mpad, a.N, device_cus());
+  // The smaller tiles copy the token scales 16 bytes at a time; callers' own scales may be aligned to 4 bytes only.
+  const bool sa16 = (reinterpret_cast<uintptr_t>(a.sa) & 15) == 0;
+  const TileId tile = sa16 ? plan_tile(a.M, a.Mpad, a.N, device_cus()) : kTile256;
   if (tile != kTile256) return launch_gemm_tiles(a, tile, stream);
   const int wide = prefill_wide_columns(a.Mpad, a.N, device_cus());
   if (wide >= a.N) return launch_dense<4>(a, stream);

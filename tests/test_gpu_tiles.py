@@ -69,3 +69,14 @@ def test_channel_tiles(m, n, k):
     odd = torch.empty(m, n + 1, dtype=torch.bfloat16, device="cuda")[:, :n]  # rows that take no wide stores
     ops.channel_gemm(q, sa, w, sw, bias, out=odd)
     assert torch.equal(odd.view(torch.int16), out[:m, :n].view(torch.int16))
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 500, 384), (300, 6144, 256), (1000, 4090, 128)])
+def test_token_scales_aligned_to_four_bytes(m, n, k):
+    """Quantized activations whose scales start one float into a buffer: the same bits as aligned ones."""
+    w, s = synth.weight(n, k, seed=3, device="cuda")
+    q, sa = ops.act_quant(synth.activations(m, k, seed=4).cuda(), m_pad=ops.plan(m, n, k)[1])
+    odd = torch.empty(sa.numel() + 1, device="cuda")[1:].view_as(sa).copy_(sa)
+    assert odd.data_ptr() % 16 == 4 and odd.is_contiguous()
+    want = ops.block_fp8_gemm_q(q, sa, m, w, s).view(torch.int16)
+    assert torch.equal(ops.block_fp8_gemm_q(q, odd, m, w, s).view(torch.int16), want)
