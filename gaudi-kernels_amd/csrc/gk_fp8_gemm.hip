@@ -547,15 +547,11 @@ static hipError_t decode_token_channel_launch(const GemmArgs& a, hipStream_t str
 }
 
 hipError_t launch_gemm_decode(const GemmArgs& a, hipStream_t stream) {
-  // 33 .. 48 tokens leave the fourth tile of the 64-row layout empty: three tiles read and multiply a quarter less
-  // (every workgroup reads all tiles; the activations' L2 reads and the weights' HBM reads add up in a CU).  The same
-  // bits.  M = 40, N = 4096, K = 14336: 21.4 -> 18.3 us.
-  const int mt = a.dec.mt == 4 && a.M <= 48 ? 3 : a.dec.mt;
-  switch (decode_key(a.dec.nw, a.dec.r, a.dec.u, mt)) {
+  const DecodeShape d = launched_shape(a.dec, a.M);
+  switch (decode_key(d.nw, d.r, d.u, d.mt)) {
 #define GK_CASE(NW, R, U, MT) \
   case decode_key(NW, R, U, MT): return decode_launch<NW, R, U, MT>(a, stream);
     GK_DECODE_SHAPES(GK_CASE)
-    GK_DECODE_SHAPES3(GK_CASE)
 #undef GK_CASE
     default: return hipErrorInvalidValue;
   }

@@ -28,6 +28,13 @@ int main() {
           // gk_fp8_block_gemm_bf16 / _q_bf16: make_plan's decode shape
           const DecodeShape d = gk::fit_group_step(gk::plan_decode_shape(n, g, packed != 0, mt), g);
           check(d, 3, "block gemm", n, g, mt, packed);
+          // as launched: the fewest and the most tokens of the plan, and either side of three tiles
+          for (int m : {mt == 4 ? 33 : 1, 48, 49, 64})
+            if (m <= 16 * mt) check(gk::launched_shape(d, m), 3, "block gemm, launched", n, g, mt, packed);
+          if (gk::launched_shape(d, 16 * mt).mt != mt || gk::launched_shape(d, 33).mt != (mt == 4 ? 3 : mt)) {
+            ++bad;
+            std::printf("launched_shape: mt=%d\n", mt);
+          }
           // the fused-quantizer form (one token tile)
           if (mt == 1) check(gk::fused_quant_shape(d, g), 3, "block gemm, fused quantizer", n, g, mt, packed);
         }

@@ -2,7 +2,7 @@
 
 gaudi-kernels_amd/csrc/gk_fp8_plan.h holds the planner and the instantiation
 lists the dispatch switches over; tests/csrc/plan_check.cpp runs the planner
-over the N tiers, G = 1..256 groups, 1/2/4 token tiles and both weight
+over the N tiers, G = 1..256 groups, 1/2/4 token tiles (as launched, too: a four-tile plan may run three) and both weight
 layouts (with g++, no GPU) and checks each result against its list.  A shape
 missing there would make the GEMM entry points return GK_DEVICE_ERROR for a
 plan gk_fp8_block_gemm_plan reports as valid.  The same program checks that
