@@ -253,7 +253,7 @@ def block_fp8_gemm(x, weight, scales, bias=None, *, native_half=False, variant=N
     _, _, ws_bytes = plan(m, n, k, flags, w8)
     ws = _checked_workspace(workspace, ws_bytes, device)
     if out is None:
-        out = x.new_empty((m, n))
+        out = torch.empty(m, n, dtype=torch.bfloat16, device=device)
     elif out.dtype != torch.bfloat16 or out.shape != (m, n) or out.stride(1) != 1 or out.device != device:
         raise ValueError("out must be bf16 [M, N] with unit column stride on the same GPU")
     lib = nat.load()

@@ -352,3 +352,14 @@ def test_prefill_two_tile_widths(m, n, native_half):
     rows = torch.randperm(m, generator=torch.Generator().manual_seed(3))[:40].sort().values
     ref = block_fp8.reference(x[rows], w, s, native_half=native_half, bias=bias)
     assert_parity(y[rows.cuda()].cpu(), ref, f"two widths {m}x{n}")
+
+
+def test_output_is_a_plain_tensor():
+    """x of a tensor subclass: the operation allocates a plain tensor, not one of x's class."""
+    class Sub(torch.Tensor):
+        pass
+
+    x = synth.activations(3, 256, seed=1).cuda()
+    w, s = synth.weight(128, 256, seed=2, device="cuda")
+    y = ops.block_fp8_gemm(x.as_subclass(Sub), w, s)
+    assert type(y) is torch.Tensor and torch.equal(y.view(torch.int16), ops.block_fp8_gemm(x, w, s).view(torch.int16))
