@@ -36,3 +36,10 @@ def test_threads_and_streams():
     for th in threads:
         th.join()
     assert not wrong
+
+
+def test_stream_handle_is_the_current_stream():
+    device = torch.device("cuda", torch.cuda.current_device())
+    for stream in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(stream):
+            assert ops._stream(device) == stream.cuda_stream
