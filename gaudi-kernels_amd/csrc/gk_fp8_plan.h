@@ -149,37 +149,67 @@ inline int prefill_wide_columns(int Mpad, int N, int cus, double* rounds_out = n
 // the LDS of two workgroups on a CU (shorter stages), the others use it whole.
 enum TileId { kTile64x32 = 0, kTile64x64, kTile128x64, kTile128x64Two, kTile128x128, kTile256 };
 
-// Which tile: the least estimated time, rounds over the CUs times the time of
-// one 128-K group in a round.  That time, measured on MI355X (us a group and
-// round; bits are the same for every tile): 64 x 32 0.27, 64 x 64 0.29, 128 x 64
-// 0.46, 128 x 128 0.73, 256 x 256 1.42 on an almost empty chip and 1.66 with all
-// CUs busy; with two workgroups on a CU 128 x 64 0.40 a tile.
-// M = 300, N = 6144, K = 4096: 49.8 us in 48 tiles of 256 x 256, 18.2 us in 240
-// tiles of 128 x 64; M = 1024, N = K = 4096: 49.2 and 26.4 us (128 x 128); M =
-// 1024, N = 28672: 143 us in 256 x 256 tiles, 172 us in 128 x 128 ones.
-inline TileId plan_tile(int M, int Mpad, int N, int cus) {
+// What a group of 128 K costs: E4M3 codes with block scales, the same with the
+// half-range conversion of every weight fragment, per-token / per-channel (no
+// promotion).
+enum TileForm { kFormOcp = 0, kFormHalf, kFormChannel };
+
+// Estimated us of one round over the CUs: round + G (group + busy f) + loose,
+// f the share of the CUs that the rounds fill, busy_more in the place of busy
+// when there is more than one round, loose only where the output rows take no
+// wide stores (16 bytes for the 256 x 256 tile, 8 for the others).
+struct TileCost {
+  double round, group, busy, busy_more, loose;
+};
+
+// Which tile: the least estimated time.  The costs are fitted to 3587 measured
+// calls on MI355X (all tiles at 65 <= M <= 16384, 256 <= N <= 32768, 256 <= K <=
+// 14336, odd N among them; bits are the same for every tile).  Over these the
+// chosen tile takes 1.010 (half range 1.001, per-channel 1.007) times the best
+// one's time; one set of costs for all three forms, counted in groups alone,
+// took 1.016, 1.005 and 1.035 and was up to 15% slower than 256 x 256 tiles where
+// it chose others (half range M = 700, N = 6144, K = 14336 308 us against 293;
+// M = 4096, N = K = 2048 33.0 against 29.6).
+// M = 300, N = 6144, K = 4096: 49.8 us in 48 tiles of 256 x 256, 17.6 us in 240
+// tiles of 128 x 64; M = 1024, N = K = 4096: 47.1 and 25.2 us (128 x 128); M =
+// 1024, N = 28672: 107 us in 256 x 256 tiles, 172 us in 128 x 128 ones.
+inline TileId plan_tile(int M, int Mpad, int N, int cus, int G = 32, TileForm form = kFormOcp, bool rows16 = true,
+                        bool rows8 = true) {
   if (cus <= 0) return kTile256;
-  auto rounds = [&](long long bn, long long bm) {
-    const long long tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-    return static_cast<double>((tiles + cus - 1) / cus);
+  static constexpr TileCost kCosts[3][6] = {
+      {{2.9, 0.205, 0, 0, 0.3}, {3.05, 0.24, 0, 0, 0.6}, {3.75, 0.335, 0, 0, 0.85},
+       {2.4, 0.30, 0, 0.018, 1.25}, {4.55, 0.53, 0.113, 0.26, 2.75}, {10.4, 1.11, 0.49, 0.49, 7.1}},
+      {{2.7, 0.56, 0, 0, 0.3}, {2.9, 0.615, 0, 0, 0.6}, {3.8, 1.055, 0, 0, 0.8},
+       {2.4, 0.925, 0, 0, 0.9}, {4.8, 1.235, 0.075, 0.15, 1.8}, {8.3, 2.53, 0.395, 0.395, 6.9}},
+      {{2.95, 0.135, 0, 0, 0.4}, {3.5, 0.175, 0, 0, 0.6}, {4.7, 0.28, 0, 0, 1.05},
+       {3.0, 0.294, 0, 0, 1.07}, {7.7, 0.355, 0.158, 0.145, 2.5}, {8.9, 1.0, 0.4, 0.4, 27.0}}};
+  // Weights past the 256 MB last-level cache come from HBM in every call; fewer tokens a tile, more fetches of a panel.
+  static constexpr double kCold[6] = {1.3, 1.3, 1.3, 1.3, 1.15, 1.05};
+  const bool cold = static_cast<long long>(N) * G * 128 > (1LL << 28);
+  auto cost = [&](TileId t, double rounds, double tiles, bool wide) {
+    const TileCost& c = kCosts[form][t];
+    const double f = tiles / cus / rounds;
+    const double us = rounds * (c.round + G * (c.group + (rounds > 1.0 ? c.busy_more : c.busy) * f) + (wide ? 0.0 : c.loose));
+    return cold ? us * kCold[t] : us;
   };
-  double best = 0.0;
-  prefill_wide_columns(Mpad, N, cus, &best);
+  double rounds256 = 0.0;
+  prefill_wide_columns(Mpad, N, cus, &rounds256);
   const double tiles256 = static_cast<double>(Mpad / 256) * ((N + 255LL) / 256);
-  best *= 1.42 + 0.24 * (tiles256 < cus ? tiles256 / cus : 1.0);
+  double best = cost(kTile256, rounds256, tiles256 < cus ? tiles256 : cus, rows16);
   TileId id = kTile256;
-  auto offer = [&](TileId t, double cost) {
-    if (cost < best) {
-      best = cost;
+  auto offer = [&](TileId t, long long bn, long long bm) {
+    const long long tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    if (tiles > cus && t == kTile128x64) t = kTile128x64Two;  // two workgroups a CU
+    const double us = cost(t, static_cast<double>((tiles + cus - 1) / cus), static_cast<double>(tiles), rows8);
+    if (us < best) {
+      best = us;
       id = t;
     }
   };
-  const double r6432 = rounds(64, 32), r6464 = rounds(64, 64), r12864 = rounds(128, 64);
-  offer(kTile128x128, 0.73 * rounds(128, 128));
-  if (r12864 <= 1.0) offer(kTile128x64, 0.46);
-  else offer(kTile128x64Two, 0.40 * r12864);
-  offer(kTile64x64, 0.29 * r6464);
-  offer(kTile64x32, 0.27 * r6432);
+  offer(kTile128x128, 128, 128);
+  offer(kTile128x64, 128, 64);
+  offer(kTile64x64, 64, 64);
+  offer(kTile64x32, 64, 32);
   return id;
 }
 

@@ -813,6 +813,14 @@ hipError_t launch_dense(const GemmArgs& a, hipStream_t stream) {
 
 }  // namespace
 
+// plan_tile for these operands: whether the output rows take 16-byte and 8-byte stores.
+static TileId tile_for(const GemmArgs& a, int mpad, TileForm form) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(a.yp ? static_cast<const void*>(a.yp) : a.y);
+  const bool rows16 = (p & 15) == 0 && (a.yp ? a.ldyp % 4 == 0 : a.ldy % 8 == 0);
+  const bool rows8 = a.yp ? rows16 : (p & 7) == 0 && a.ldy % 4 == 0;  // fp32 partials: 16 bytes in both kernels
+  return plan_tile(a.M, mpad, a.N, device_cus(), a.G, form, rows16, rows8);
+}
+
 // Per-token / per-channel form: a.qa row-major [M][a.ldq], a.sa [M], a.sw [N]; any M.
 hipError_t launch_gemm_channel256(const GemmArgs& a, hipStream_t stream) {
   if (static_cast<int64_t>(256) * a.ldq > int64_t{0xffffffff} || static_cast<int64_t>(256) * a.K > int64_t{0xffffffff})
@@ -821,7 +829,7 @@ hipError_t launch_gemm_channel256(const GemmArgs& a, hipStream_t stream) {
   if (e != hipSuccess) return e;
   GemmArgs c = a;
   c.Mpad = (a.M + kBM - 1) / kBM * kBM;
-  const TileId tile = plan_tile(a.M, c.Mpad, a.N, device_cus());
+  const TileId tile = tile_for(a, c.Mpad, kFormChannel);
   if (tile != kTile256) return launch_gemm_tiles(c, tile, stream);
   const int wide = prefill_wide_columns(c.Mpad, a.N, device_cus());
   if (wide < a.N) return launch_split<false, false, true>(c, wide, stream);
@@ -842,7 +850,7 @@ hipError_t launch_gemm_prefill256(const GemmArgs& a, hipStream_t stream) {
   if (a.Mpad % kBM != 0 || !prefill256_fits(a)) return hipErrorInvalidValue;
   // The smaller tiles copy the token scales 16 bytes at a time; callers' own scales may be aligned to 4 bytes only.
   const bool sa16 = (reinterpret_cast<uintptr_t>(a.sa) & 15) == 0;
-  const TileId tile = sa16 ? plan_tile(a.M, a.Mpad, a.N, device_cus()) : kTile256;
+  const TileId tile = sa16 ? tile_for(a, a.Mpad, a.half_w ? kFormHalf : kFormOcp) : kTile256;
   if (tile != kTile256) return launch_gemm_tiles(a, tile, stream);
   const int wide = prefill_wide_columns(a.Mpad, a.N, device_cus());
   if (wide >= a.N) return launch_dense<4>(a, stream);

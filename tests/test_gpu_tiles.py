@@ -47,11 +47,11 @@ def test_tiles_equal_256_rows(m, n, k):
     assert torch.equal(ops.block_fp8_gemm(x[:m], w, s).view(torch.int16), big[:m].view(torch.int16))
 
 
-# 64x32, 64x64, 128x64, 128x64 twice a CU, 128x128, 256x256 in one range and (last) in two of 256 and 192 columns
+# 64x32, 64x64, 128x64, 128x64 twice a CU (two), 128x128, 256x256 in one range and (last) in two of 256 and 192 columns
 @pytest.mark.parametrize("m,n,k", [(17, 500, 384), (128, 6140, 640), (300, 6144, 256), (777, 5003, 384),
-                                   (1000, 4090, 128), (2047, 7168, 256), (4095, 7160, 256)])
+                                   (1000, 4090, 128), (640, 4090, 2048), (2047, 7168, 256), (4095, 7160, 256)])
 def test_channel_tiles(m, n, k):
-    """Every tile of the per-channel GEMM against 64-bit products: P is a sum of at most 640 exact products whose
+    """Every tile of the per-channel GEMM against 64-bit products: P is a sum of at most 2048 exact products whose
     fp8 matrix instruction sums to within 1e-4 of its scale; the rest is three fp32 roundings and the bf16 one."""
     gen = torch.Generator(device="cuda").manual_seed(m)
     q, sa = ops.token_quant(torch.randn(m, k, generator=gen, device="cuda").bfloat16())
