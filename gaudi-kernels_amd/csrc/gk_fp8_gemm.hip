@@ -611,7 +611,8 @@ hipError_t launch_gemm_generic(const GemmArgs& a, hipStream_t stream) {
   const int64_t tiles_n = (a.N + 31LL) / 32;
   if (a.M <= 16) return generic_launch<1, 8>(a, 1, tiles_n, stream);
   const int64_t tiles_m = (a.M + 31LL) / 32, tiles = tiles_m * tiles_n;
-  return tiles <= 256 ? generic_launch<2, 8>(a, tiles_m, tiles, stream) : generic_launch<2, 4>(a, tiles_m, tiles, stream);
+  return tiles <= device_cus() ? generic_launch<2, 8>(a, tiles_m, tiles, stream)
+                               : generic_launch<2, 4>(a, tiles_m, tiles, stream);
 }
 
 }  // namespace gk

@@ -287,6 +287,9 @@ struct GemmArgs {
   float* swiglu_s = nullptr;
 };
 
+// Compute units of the current device (cached per device; 0 if unknown).  gk_fp8_prefill.hip.
+int device_cus();
+
 hipError_t launch_gemm_decode(const GemmArgs& a, hipStream_t stream);
 hipError_t launch_gemm_prefill(const GemmArgs& a, hipStream_t stream);     // dispatches by M
 hipError_t launch_gemm_prefill256(const GemmArgs& a, hipStream_t stream);  // 256 x 256 tiles, Mpad % 256 == 0

@@ -220,7 +220,7 @@ hipError_t launch_rms_norm(const uint16_t* x, const uint16_t* res, int64_t ld_in
   // nothing hides while there are at most as many rows as CUs: then a row takes one pass, with 512 or 1024 threads
   // beyond 2048 columns.  More rows hide it themselves and keep 256 threads (16 x 4096 with residual and quantizer:
   // 4.2 -> 3.7 us, 16 x 7168 5.8 -> 4.6; 4093 x 4096 24.4 us either way).
-  const int nt = grid > 256 || width <= 8 * 256 ? 256 : width <= 8 * 512 ? 512 : 1024;
+  const int nt = grid > static_cast<unsigned>(device_cus()) || width <= 8 * 256 ? 256 : width <= 8 * 512 ? 512 : 1024;
 #define GK_NORM_T(NT, PASSES, A, Q, H, P, V)                                                               \
   rms_norm_kernel<NT, PASSES, A, Q, H, P, V><<<grid, NT, 0, stream>>>(x, res, ld_in, gamma, rows, width, eps, off, \
                                                                       res_out, norm_out, ld_out, q, sa, Mpad)

@@ -718,6 +718,9 @@ __global__ __launch_bounds__(512) void gemm_prefill256_split_kernel(
 // The 160 KB of dynamic LDS is above the default limit: raise it once per device.
 constexpr int kMaxDevices = 64;
 
+std::once_flag g_cu_once[kMaxDevices];
+int g_cus[kMaxDevices];
+
 std::once_flag g_lds_once[kMaxDevices][41];
 hipError_t g_lds_err[kMaxDevices][41];
 
@@ -771,20 +774,6 @@ hipError_t launch_split(const GemmArgs& a, int wide, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Compute units of the current device (cached per device; 0 if unknown).
-std::once_flag g_cu_once[kMaxDevices];
-int g_cus[kMaxDevices];
-
-int device_cus() {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
-  std::call_once(g_cu_once[dev], [dev] {
-    int n = 0;
-    g_cus[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess ? n : 0;
-  });
-  return g_cus[dev];
-}
-
 template <bool HALF, bool GROUPED, bool WPACK = false, int NA = 4, bool SWI = false>
 hipError_t launch256(const GemmArgs& a, const int32_t* group_off, const int32_t* group_cnt, int n_groups,
                      int64_t w_stride, int64_t sw_stride, int kparts, float* yp, int64_t ldyp, hipStream_t stream) {
@@ -812,6 +801,16 @@ hipError_t launch_dense(const GemmArgs& a, hipStream_t stream) {
 
 
 }  // namespace
+
+int device_cus() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  std::call_once(g_cu_once[dev], [dev] {
+    int n = 0;
+    g_cus[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess ? n : 0;
+  });
+  return g_cus[dev];
+}
 
 // plan_tile for these operands: whether the output rows take 16-byte and 8-byte stores.
 static TileId tile_for(const GemmArgs& a, int mpad, TileForm form) {
