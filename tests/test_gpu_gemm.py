@@ -214,9 +214,9 @@ def test_output_padding_untouched():
 
 @pytest.mark.parametrize("m,n", [(300, 203), (256, 200), (40, 1000)])
 def test_prefill_epilogue_forms_same_bits(m, n):
-    """The prefill tile leaves through LDS as whole-row 16-byte stores when y is 16-byte aligned with a row stride
-    that is a multiple of 8, and through per-fragment stores otherwise: both forms write the same bits, only
-    inside [M, N] (a ragged last 16-byte chunk included), and match the oracle."""
+    """The prefill variant at shapes of its small tiles (64 x 32), which store 8 bytes a lane where the row allows it
+    and single values otherwise: every row alignment writes the same bits, only inside [M, N] (a ragged last chunk
+    included), and matches the oracle.  (test_gpu_prefill256.py: the output forms of the 256 x 256 tile.)"""
     k = 512
     w, s = synth.weight(n, k, seed=n + 3)
     x = synth.activations(m, k, seed=m + 4)
@@ -333,8 +333,9 @@ def test_decode_two_tile_narrow_step_shape(m, n, k):
 @pytest.mark.parametrize("m,n,native_half", [(4096, 7168, False), (3000, 6000, True)])
 def test_prefill_two_tile_widths(m, n, native_half):
     """GEMMs whose 256 x 256 tiles need more than one round over the CUs run their last columns in 192-wide tiles
-    (a second launch).  Those columns must equal, bit for bit, a separate GEMM over just those columns (256-wide
-    tiles), for row-major and packed weights, and meet the gate against the oracle on sampled rows."""
+    (one launch of two ranges).  Those columns must equal, bit for bit, a separate GEMM over just those columns (few
+    enough for 128 x 128 or 256 x 256 tiles), for row-major and packed weights, and meet the gate against the oracle on
+    sampled rows."""
     k = 1024
     w, s = synth.weight(n, k, seed=n + 5)
     x = synth.activations(m, k, seed=m + 5)
@@ -343,7 +344,7 @@ def test_prefill_two_tile_widths(m, n, native_half):
     y = ops.block_fp8_gemm(xd, wd, sd, bd, native_half=native_half)
     yp = ops.block_fp8_gemm(xd, ops.pack_weight(wd), sd, bd, native_half=native_half)
     assert torch.equal(y.view(torch.int16), yp.view(torch.int16))
-    # the narrow tiles take the columns from the last multiple of 256 that keeps the first launch in whole
+    # the narrow tiles take the columns from the last multiple of 256 that keeps the first range in whole
     # rounds (4096 and 2048 here); compare the columns from a multiple of 128 inside the narrow range
     c0 = (n - 1024) // 128 * 128
     ys = ops.block_fp8_gemm(xd, wd[c0:].contiguous(), sd[c0 // 128:].contiguous(), bd[c0:].contiguous(),

@@ -14,7 +14,8 @@ from oracle import block_fp8, synth
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(1, 1, 1), (1, 31, 127), (16, 33, 129), (17, 32, 1000), (33, 65, 1025), (40, 129, 2880)]
+# the last: 297 workgroups, more than the CUs (four waves each, two partial sums a wave)
+SHAPES = [(1, 1, 1), (1, 31, 127), (16, 33, 129), (17, 32, 1000), (33, 65, 1025), (40, 129, 2880), (257, 1030, 1395)]
 
 
 @pytest.mark.parametrize("m,n,k", SHAPES)

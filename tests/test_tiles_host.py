@@ -40,6 +40,8 @@ FORM_CASES = [
     ((65, 500, 384, OCP, 1), 0), ((128, 6140, 640, OCP, 1), 1), ((300, 6144, 640, OCP, 1), 2),
     ((777, 5003, 384, OCP, 0), 3), ((1000, 4090, 896, OCP, 1), 4), ((4096, 6144, 256, OCP, 1), 5),
     ((4096, 6144, 8320, OCP, 1), 5), ((4096, 6144, 384, OCP, 1), 5), ((4096, 6144, 128, OCP, 1), 5),
+    *(((m, n, k, form, wide), 5) for m, n in ((2040, 7163), (3000, 6001)) for k in (1152, 256, 384, 512)
+      for form in (OCP, HALF) for wide in (0, 1)),  # test_gpu_prefill256.py
     ((65, 500, 384, HALF, 1), 0), ((128, 6140, 640, HALF, 1), 1), ((300, 6144, 640, HALF, 1), 2),
     ((777, 5003, 384, HALF, 0), 3), ((1000, 4090, 896, HALF, 1), 4),
     ((17, 500, 384, CHANNEL, 1), 0), ((128, 6140, 640, CHANNEL, 1), 1), ((300, 6144, 256, CHANNEL, 1), 2),
@@ -54,3 +56,13 @@ def test_plan_tile_forms(tmp_path):
     out = subprocess.run([str(exe)], input="\n".join(" ".join(map(str, c)) for c, _ in FORM_CASES), check=True,
                          capture_output=True, text=True).stdout.split()
     assert [(c, int(v)) for (c, _), v in zip(FORM_CASES, out)] == FORM_CASES
+
+
+def test_column_ranges(tmp_path):
+    """test_gpu_prefill256.py: one column range of 256-wide tiles, and two."""
+    (tmp_path / "p.cpp").write_text("""#include "gk_fp8_plan.h"
+int main() { return gk::prefill_wide_columns(2048, 7163, 256) == 7163 && gk::prefill_wide_columns(3072, 6001, 256) == 2048 ? 0 : 1; }
+""")
+    exe = tmp_path / "p"
+    subprocess.run(["g++", "-std=c++17", "-I", str(CSRC), str(tmp_path / "p.cpp"), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)]).returncode == 0
