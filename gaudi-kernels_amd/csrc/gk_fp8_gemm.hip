@@ -558,10 +558,9 @@ hipError_t launch_gemm_decode(const GemmArgs& a, hipStream_t stream) {
 }
 
 hipError_t launch_gemm_prefill(const GemmArgs& a, hipStream_t stream) {
-  // 256 x 256 tiles (gk_fp8_prefill.hip) at every M > 16: they skip the 32-row
-  // blocks past M.  (A 128 x 128 kernel measured 1.2-3x slower at 16 < M <= 128
-  // on MI355X.)  The plan sends shapes whose panels exceed the kernel's 32-bit
-  // offsets to the generic variant.
+  // The LDS-tiled kernels (256 x 256 tiles, or smaller ones by plan_tile).  The
+  // plan sends shapes whose panels exceed their 32-bit offsets to the generic
+  // variant.
   if (!prefill256_fits(a)) return hipErrorInvalidValue;
   return launch_gemm_prefill256(a, stream);
 }

@@ -101,7 +101,8 @@ __device__ inline uint4 act_mul8(uint4 gv, uint4 uv) {
 
 // Row padding of the quantized-activation workspace.
 constexpr int kDecodeMaxRows = 16;   // one MFMA column tile of tokens (the fused quantizer, per-channel decode)
-constexpr int kDecodeMaxTokens = 64;  // decode variant: M <= 64 in 1, 2 or 4 column tiles (Mpad = 16, 32, 64)
+// decode variant: M <= 64 in 1, 2 or 4 column tiles (Mpad = 16, 32, 64), of which 33 .. 48 tokens compute three
+constexpr int kDecodeMaxTokens = 64;
 // Token tiles of the decode variant for M tokens (Mpad = 16 * decode_tiles(M)).
 inline int decode_tiles(int64_t M) { return M <= 16 ? 1 : M <= 32 ? 2 : 4; }
 // Offset of codes byte `e` (0..127) of token `row` in group g of the decode fragment layout with Mpad rows:
@@ -260,13 +261,13 @@ struct GemmArgs {
   // codes, sa [M] per token, sw [N] per output channel, no per-group promotion.
   bool channel = false;
   int64_t ldq = 0;
-  // Weights in the fragment-packed layout of launch_pack_weight (decode and
-  // 256 x 256 kernels only).
+  // Weights in the fragment-packed layout of launch_pack_weight (not the
+  // generic kernel).
   bool wpack = false;
   // Decode variant only: qa is the bf16 activation x [M][ldq] (16-byte
   // aligned rows, ldq % 8 == 0), quantized inside the GEMM (sa unused).
   bool xq = false;
-  // K range of a larger weight (decode and 256 x 256 kernels, block scaling):
+  // K range of a larger weight (not the generic kernel; block scaling):
   // w and sw already point at the range's first group, G counts its groups,
   // K stays the weight row stride and gs the groups of the whole row (the
   // scale-grid row stride and, for packed weights, the 16-row tile stride in
@@ -291,9 +292,11 @@ struct GemmArgs {
 int device_cus();
 
 hipError_t launch_gemm_decode(const GemmArgs& a, hipStream_t stream);
-hipError_t launch_gemm_prefill(const GemmArgs& a, hipStream_t stream);     // dispatches by M
-hipError_t launch_gemm_prefill256(const GemmArgs& a, hipStream_t stream);  // 256 x 256 tiles, Mpad % 256 == 0
-// Smaller tiles of the same GEMM (gk_fp8_tiles.hip): the same conditions, the same result bits.  Also the channel form.
+hipError_t launch_gemm_prefill(const GemmArgs& a, hipStream_t stream);
+// 256 x 256 tiles, or smaller ones where plan_tile says so; Mpad % 256 == 0.
+hipError_t launch_gemm_prefill256(const GemmArgs& a, hipStream_t stream);
+// Smaller tiles of the same GEMM (gk_fp8_tiles.hip): the same conditions and a.sa 16-byte aligned, the same result
+// bits.  Also the channel form.
 hipError_t launch_gemm_tiles(const GemmArgs& a, TileId tile, hipStream_t stream);
 // The 256 x 256 kernels address a 256-row weight panel and the whole
 // group-major activation array with 32-bit byte offsets.
@@ -301,7 +304,6 @@ inline bool prefill256_fits(const GemmArgs& a) {
   return static_cast<int64_t>(a.Mpad) * a.G * 128 <= int64_t{0xffffffff} &&
          static_cast<int64_t>(256) * a.K <= int64_t{0xffffffff};
 }
-// Grouped (MoE) 256 x 256 GEMM over expert row segments; see gk_fp8_prefill.hip.
 // Grouped (MoE) 256 x 256 GEMM over expert row segments (gk_fp8_prefill.hip):
 // segment e starts at group_off[e] (multiple of 256) and holds group_cnt[e]
 // live rows; 32-row blocks past the live rows are skipped.  yp == nullptr:
@@ -312,11 +314,11 @@ hipError_t launch_gemm_grouped256(const GemmArgs& a, const int32_t* group_off, c
                                   int n_groups, int kparts, float* yp, hipStream_t stream);
 hipError_t launch_gemm_generic(const GemmArgs& a, hipStream_t stream);
 // Per-token / per-channel GEMM (a.channel): M <= 16 streams weights (decode
-// shapes), larger M runs the 256 x 256 kernel in its channel form.
+// shapes), larger M runs the LDS-tiled kernels in their channel form (tiles by plan_tile).
 hipError_t launch_gemm_channel(const GemmArgs& a, hipStream_t stream);
 // Per-token quantizer fused into the per-channel decode: a.qa = bf16 x [M][a.ldq], M <= 16.
 hipError_t launch_gemm_token_channel(const GemmArgs& a, hipStream_t stream);
-hipError_t launch_gemm_channel256(const GemmArgs& a, hipStream_t stream);  // gk_fp8_prefill.hip
+hipError_t launch_gemm_channel256(const GemmArgs& a, hipStream_t stream);  // its M > 16; gk_fp8_prefill.hip
 
 // ---- row-parallel completion (gk_fp8_reduce.hip) -------------------------------------
 // rank_sum.c:4-42: dst[i] = sum over r < world of gathered[r * elems + i] in

@@ -1,6 +1,6 @@
 // Device helpers of the kernels that stage operand tiles in LDS with
 // direct-to-LDS buffer loads and read MFMA fragments from it with inline-asm
-// ds_read (gk_fp8_prefill.hip).
+// ds_read (gk_fp8_prefill.hip, gk_fp8_tiles.hip).
 #pragma once
 
 #include <type_traits>

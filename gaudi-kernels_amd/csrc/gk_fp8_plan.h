@@ -170,9 +170,10 @@ struct TileCost {
 // took 1.016, 1.005 and 1.035 and was up to 15% slower than 256 x 256 tiles where
 // it chose others (half range M = 700, N = 6144, K = 14336 308 us against 293;
 // M = 4096, N = K = 2048 33.0 against 29.6).
-// M = 300, N = 6144, K = 4096: 49.8 us in 48 tiles of 256 x 256, 17.6 us in 240
+// M = 300, N = 6144, K = 4096: 45.3 us in 48 tiles of 256 x 256, 15.6 us in 240
 // tiles of 128 x 64; M = 1024, N = K = 4096: 47.1 and 25.2 us (128 x 128); M =
-// 1024, N = 28672: 107 us in 256 x 256 tiles, 172 us in 128 x 128 ones.
+// 1024, N = 28672: 106 us in 256 x 256 tiles, 162 us in 128 x 128 ones (us of the
+// launch, launches back to back).
 inline TileId plan_tile(int M, int Mpad, int N, int cus, int G = 32, TileForm form = kFormOcp, bool rows16 = true,
                         bool rows8 = true) {
   if (cus <= 0) return kTile256;

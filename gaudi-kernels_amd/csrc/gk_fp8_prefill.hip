@@ -764,8 +764,8 @@ hipError_t launch_split(const GemmArgs& a, int wide, hipStream_t stream) {
   const int split = tiles_m * (wide / 256);
   const unsigned blocks = static_cast<unsigned>(split + tiles_m * ((n2 + 191) / 192));
   // Columns [wide, N): weight rows from `wide` (row-major: + wide * K bytes; packed:
-  // 16-row tiles of gs * 2048 = K * 16 bytes, the same offset), scale rows from wide / 128.
-  // (per-channel scales: one per column).
+  // 16-row tiles of gs * 2048 = K * 16 bytes, the same offset), scale rows from
+  // wide / 128 (per-channel scales: one per column).
   gemm_prefill256_split_kernel<HALF, WPACK, CH><<<blocks, 512, kLdsBytes, stream>>>(
       split, a.qa, a.sa, a.ldy, a.M, a.K, a.G, a.Mpad, a.ldq, a.gstride(), a.ldyp, a.accumulate ? 1 : 0, a.w, a.sw,
       a.bias, a.y, a.yp, wide, a.w + static_cast<int64_t>(wide) * a.K,
@@ -841,10 +841,10 @@ hipError_t launch_gemm_channel256(const GemmArgs& a, hipStream_t stream) {
 
 // Requires K % 128 == 0, 16-byte aligned weights, Mpad % 256 == 0 (qa/sa
 // padded with zero rows up to Mpad).  Shapes that 256 x 256 tiles would spread
-// over too few CUs run smaller tiles (plan_tile, gk_fp8_tiles.hip).  Large GEMMs may run in two column
-// ranges of different tile widths (prefill_wide_columns), in one launch; each
-// output column is computed by one workgroup either way, with the same
-// per-element arithmetic.
+// over too few CUs run smaller tiles (plan_tile, gk_fp8_tiles.hip).  Large GEMMs
+// may run in two column ranges of different tile widths (prefill_wide_columns),
+// in one launch; each output column is computed by one workgroup either way,
+// with the same per-element arithmetic.
 hipError_t launch_gemm_prefill256(const GemmArgs& a, hipStream_t stream) {
   if (a.Mpad % kBM != 0 || !prefill256_fits(a)) return hipErrorInvalidValue;
   // The smaller tiles copy the token scales 16 bytes at a time; callers' own scales may be aligned to 4 bytes only.

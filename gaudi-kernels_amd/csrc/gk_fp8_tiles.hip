@@ -7,12 +7,13 @@
 // sw[n / 128, g] and added in fp32, groups in ascending order -- so the result
 // bits do not depend on which of the two kernels runs, nor on the tile.
 //
-// Measured on MI355X (us, 256 x 256 tiles -> here): M = 300, N = 6144, K = 4096
-// 49.8 -> 18.2; M = 128, same weights 48.6 -> 13.0; M = 256, N = 4096, K = 3584
-// 42.8 -> 11.7; M = 1024, N = K = 4096 49.2 -> 26.4.  Bound: the LDS port (128
-// bytes a cycle).  A 128 x 64 group reads 64 KB of fragments and writes 24 KB of
-// copies, 700 of the 1000 cycles that it takes; its MFMAs take 256.  Four waves
-// of larger wave tiles read less but lose more latency (18.2 -> 21.6 us).
+// Measured on MI355X (us of the GEMM launch, launches back to back; 256 x 256
+// tiles -> here): M = 300, N = 6144, K = 4096 45.3 -> 15.6; M = 128, same weights
+// 44.3 -> 11.1; M = 256, N = K = 4096 45.0 -> 11.3; M = 1024, N = K = 4096 47.1 ->
+// 25.2.  Bound: the LDS port (128 bytes a cycle).  A 128 x 64 group reads 64 KB of
+// fragments and writes 24 KB of copies, 700 of the 1000 cycles that it takes; its
+// MFMAs take 256.  Four waves of larger wave tiles read less but lose more latency
+// (18.2 -> 21.6 us).
 //
 // Structure (one workgroup = 8 waves, 4 along N x 2 along M; a wave holds
 // 16 NA weight rows x 16 MB tokens):

@@ -169,9 +169,12 @@ gk_status gk_fp8_block_gemm_plan(int64_t m, int64_t n, int64_t k, uint32_t flags
  * act_row_scale -> quant_act_fp16_1k -> dequant_weight_fp16_1k -> MME ->
  * epilogue(_bias) (fp8_hybrid_tpcsim_test.cpp:180-324).  Dispatch by M:
  * M <= 64 streams weights (decode: one to four 16-token tiles share each
- * weight fragment), larger M runs the LDS-tiled MFMA kernel (prefill).  The activations are quantized into the workspace first.  scale_rows x scale_cols must equal ceil(n/128) x ceil(k/128)
- * (GK_INCOMPATIBLE_INPUT_SIZE otherwise, as generic_fp8_glue_test.cpp:98-100).
+ * weight fragment), larger M runs the LDS-tiled MFMA kernels (prefill).  The
+ * activations are quantized into the workspace first.  scale_rows x scale_cols
+ * must equal ceil(n/128) x ceil(k/128) (GK_INCOMPATIBLE_INPUT_SIZE otherwise, as generic_fp8_glue_test.cpp:98-100).
  * bias may be NULL.  Inputs are not checked for NaN (see gk_fp8_check_inputs).
+ * Within a variant a row's result bits do not depend on the other rows or on
+ * their number.
  * GK_FLAG_WEIGHT_PACKED: w is gk_fp8_pack_weight's output for (n, k); the
  * results are bit-identical to those on the row-major weights. */
 gk_status gk_fp8_block_gemm_bf16(const void* x, int64_t m, int64_t k, int64_t ldx, const void* w, int64_t n,
@@ -370,9 +373,9 @@ gk_status gk_fp8_gelu_mul_quant_bf16(const void* gate_up, int64_t rows, int64_t 
  * stride ld_in), gamma bf16 [width] -> out bf16 [rows, width] (row stride
  * ld_out), out = bf16((x * inv) * (gamma + weight_offset)) with
  * inv = 1 / sqrt(sum(x^2) * (1/width) + epsilon) per row.  The sum of squares
- * is taken exactly (fp64, fixed order) and rounded to fp32 once; inv is
- * fp32(1 / sqrt) of the fp32 argument; the products are fp32.  As the glue:
- * epsilon must be finite and > 0 and weight_offset finite
+ * is taken in fp64 in one fixed order, whatever the number of rows, and rounded
+ * to fp32 once; inv is fp32(1 / sqrt) of the fp32 argument; the products are
+ * fp32.  As the glue: epsilon must be finite and > 0 and weight_offset finite
  * (GK_UNSUPPORTED_LAYER_CONFIGURATION), 1 <= width <= 8192 and rows >= 1
  * (GK_INCOMPATIBLE_INPUT_SIZE). */
 gk_status gk_rms_norm_bf16(const void* x, int64_t rows, int64_t width, int64_t ld_in, const void* gamma,

@@ -33,3 +33,15 @@ def test_three_token_tiles(m, n, k, half):
         assert torch.equal(ops.block_fp8_gemm_q(q, sa, m, weight, sd, native_half=half).view(torch.int16), want)
     part = ops.block_fp8_gemm_kslice(xd[:m], pk, sd, 128, k - 128, native_half=half)
     assert torch.equal(part, ops.block_fp8_gemm_kslice(xd, pk, sd, 128, k - 128, native_half=half)[:m])
+
+
+# N per decode shape as above; K = 4096 at N = 6150 quantizes inside the kernel up to M = 16
+@pytest.mark.parametrize("n,k", [(500, 2048), (4100, 1152), (6150, 4096), (24600, 256)])
+@pytest.mark.parametrize("packed", [False, True])
+def test_rows_do_not_depend_on_the_batch(n, k, packed):
+    x = synth.activations(64, k, seed=n).cuda()
+    w, s = synth.weight(n, k, seed=k, device="cuda")
+    weight = ops.pack_weight(w) if packed else w
+    big = ops.block_fp8_gemm(x, weight, s).view(torch.int16)
+    for m in (1, 5, 16, 17, 32, 49):
+        assert torch.equal(ops.block_fp8_gemm(x[:m], weight, s).view(torch.int16), big[:m])
