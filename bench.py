@@ -1,12 +1,12 @@
-"""Benchmark of the MI355X block-FP8 W8A8 GEMM (BASELINE.json metric).
+"""Benchmark of the MI355X block-FP8 W8A8 GEMM (decode bandwidth over M = 1 .. 16, prefill and MoE beside it).
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu] [--only qkv|side|prefill|mlp|moe|ceiling]
     python bench.py --profile config2 [--steps K --warmup W]       # the timed step's graphs, for rocprofv3 runs
     python bench.py --profile prefill|mlp|moe [--reps R]           # eager launches, for rocprofv3 runs
     python bench.py --rocprof-summary DIR [--steps K]              # tables of a rocprofv3 csv output
 
-Workload (one "step"): BASELINE.json configs[1] decode sweep -- one block-FP8
-GEMM at each M in {1, 2, 4, 8, 16} with N=6144, K=4096 (QKV projection),
+Workload (one "step"): the decode sweep of a QKV projection -- one block-FP8
+GEMM at each M in {1, 2, 4, 8, 16} with N=6144, K=4096,
 E4M3 weights with fp32 128x128 block scales, bf16 activations quantized per
 1x128 group inside the op, bf16 output.  Inputs are synthetic (seeded
 N(0,0.02) weights with 5% x8 blocks, N(0,1) activations with 1% x20 outlier
@@ -546,7 +546,7 @@ def main():
         rocprof_summary(args.rocprof_summary, args.steps)
         return
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
-        print("bench.py measures one GPU: this build has no multi-GPU path (under tensor parallelism each GPU "
+        print("bench.py measures one GPU: the package has no multi-GPU path (under tensor parallelism each GPU "
               "runs this GEMM on its own shard of the weights); run with --gpus 1", file=sys.stderr)
         sys.exit(2)
 

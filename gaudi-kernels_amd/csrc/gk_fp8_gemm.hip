@@ -346,7 +346,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_decode_kernel(const uint8_t* __r
 // become zero), the next group's loads in flight during the current one's
 // products.  Bound by the latency of a wave's few load rounds, so the tile is
 // small and K is split: M = 200, N = K = 2880 7.0 ms (byte loads, one output a
-// thread) -> 15.4 us.
+// thread) -> 15.5 us (the launch alone, launches back to back).
 
 // 8 E4M3 codes -> 8 bf16 values.
 __device__ inline bf16x8 widen8(uint32_t lo, uint32_t hi) {
@@ -606,7 +606,7 @@ static hipError_t generic_launch(const GemmArgs& a, int64_t tiles_m, int64_t til
 hipError_t launch_gemm_generic(const GemmArgs& a, hipStream_t stream) {
   // Up to 16 tokens fill one block; beyond, two share each weight fragment.  Eight waves split K while a CU has one
   // workgroup anyway; with more workgroups than CUs four (three workgroups a CU by registers instead of one: M = 200,
-  // N = K = 2880 19.4 -> 15.4 us; M = 20 there, 90 workgroups: 7.4 us with four waves, 6.4 with eight).
+  // N = K = 2880 19.4 -> 15.5 us; M = 20 there, 90 workgroups: 7.4 us with four waves, 6.5 with eight).
   const int64_t tiles_n = (a.N + 31LL) / 32;
   if (a.M <= 16) return generic_launch<1, 8>(a, 1, tiles_n, stream);
   const int64_t tiles_m = (a.M + 31LL) / 32, tiles = tiles_m * tiles_n;

@@ -401,7 +401,7 @@ gk_status gk_fp8_rms_norm_quant_bf16(const void* x, const void* residual, int64_
                                      void* residual_out, int64_t ld_out, void* q, float* sa, int64_t m_pad,
                                      uint32_t flags, void* stream);
 
-/* ---- block-FP8 MoE layer ------------------------------------
+/* ---- block-FP8 MoE layer --------------------------------------------------------------
  * No reference function: the reference has no MoE code for this path.  The
  * layer is build-defined from the reference's pieces (oracle/moe.py restates
  * it on the CPU): top-k (k = 1 or 2) experts per token by router logit, ties

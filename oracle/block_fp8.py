@@ -168,5 +168,5 @@ def parity(y, ref):
     return max_rel, mean_rel
 
 
-MAX_REL_TOL = 1e-2   # max|y - ref| <= 1e-2 * max|ref|  (north star)
-MEAN_REL_TOL = 2e-3  # sum|y - ref| / sum|ref| <= 2e-3    (north star)
+MAX_REL_TOL = 1e-2   # max|y - ref| <= 1e-2 * max|ref|  (the parity gate)
+MEAN_REL_TOL = 2e-3  # sum|y - ref| / sum|ref| <= 2e-3    (the parity gate)

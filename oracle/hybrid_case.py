@@ -3,7 +3,7 @@
 tests/fp8_hybrid_tpcsim_test.cpp:180-380 (cases :388-392) runs the Gaudi2 prefill chain on
 generated inputs and accepts it when every output row's bf16 relative L2 error against an FP64
 OCP reference is <= 0.01 (:378), with exact zeros on identically zero rows (:369-371).  This
-module restates, for this build's tests:
+module restates, for the tests:
 
   * the closed-form weights (:211-226: code = ((col*17 + g*31 + i*7) % 118) + 8, sign from row 0
     of x or from a parity pattern), block scales (:207) and bias (:230);
@@ -88,7 +88,7 @@ def checker(x_bits, codes, scales, b=None, scale_rule="tpc"):
     """The reference test's FP64 OCP result rounded to bf16 (:326-366), float64 [m, n].
 
     scale_rule "tpc": the test's group scale fp32(max|x| / 448), 1 for an all-zero group (:341-343);
-    "oracle": block_fp8_oracle.py:27, fp32(max(max|x|, 1e-10) * fp32(1/448)) -- the rule this build
+    "oracle": block_fp8_oracle.py:27, fp32(max(max|x|, 1e-10) * fp32(1/448)) -- the rule the library
     implements.  The two differ by at most one fp32 ulp, which flips an E4M3 code now and then (and by
     far more below 1e-10, where the oracle clamps).
     """

@@ -1,7 +1,7 @@
-"""Seeded synthetic inputs for the BASELINE.json configurations (test infrastructure only).
+"""Seeded synthetic inputs for the benchmarked configurations (test infrastructure only).
 
 The reference ships no generator for the block-FP8 path; these follow the
-build-side recipe for BASELINE.json's configs:
+recipe of the benchmarked configurations:
   * weights N(0, wstd), a seeded 5% of the 128x128 blocks scaled x8, then per
     block s = amax/D, q = e4m3fn(clamp(W/s, +-D)) with D = 448 (OCP checkpoint
     convention) or 240 (config 1, Gaudi2 half range);
@@ -51,7 +51,7 @@ def activations(m, k, seed, *, outlier_frac=0.01, device="cpu"):
 
 
 def config1():
-    """W seed 0, N(0, 0.02), D = 240; X N(0, 1) seed 1, M=4, N=K=256."""
+    """The smallest configuration: W seed 0, N(0, 0.02), D = 240; X N(0, 1) seed 1, M=4, N=K=256."""
     gen = torch.Generator().manual_seed(0)
     w = torch.randn(256, 256, generator=gen) * 0.02
     wq, s = quantize_weight(w, 240.0)

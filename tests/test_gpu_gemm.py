@@ -1,9 +1,9 @@
 """GPU block-FP8 GEMM parity against the oracle (block_fp8_oracle.py:11-46).
 
-Gate (north star): max|y - ref| <= 1e-2 * max|ref| and
+Gate: max|y - ref| <= 1e-2 * max|ref| and
 sum|y - ref| / sum|ref| <= 2e-3, on the same seeded inputs.  Covers the
 reference's golden vectors, every variant (decode / prefill / generic), the
-BASELINE.json decode shapes at full size, the prefill shape at full size through
+benchmarked decode shapes at full size, the prefill shape at full size through
 sampled rows plus size-independent properties (row permutation, exact scale
 doubling), ragged shapes with bias, native_half, and untouched output padding.
 """
@@ -114,7 +114,7 @@ def test_config3_packed_against_oracle():
 
 @pytest.mark.parametrize("native_half", [False, True])
 def test_config1_as_specified(native_half):
-    """BASELINE.json config 1 end to end on the GPU: W [256, 256] N(0, 0.02) seed 0 quantized per 128x128 block
+    """The smallest configuration end to end on the GPU: W [256, 256] N(0, 0.02) seed 0 quantized per 128x128 block
     with scale = blockmax / 240 (Gaudi2 half range), codec forward to half range and inverse back to OCP on the
     GPU, then the GEMM on the round-tripped codes against the oracle on the same codes."""
     from oracle import fp8_codec

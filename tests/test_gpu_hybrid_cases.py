@@ -4,9 +4,9 @@ Inputs: the reference generator's activations (tests/golden/hybrid_gemm_x.npz), 
 block scales and bias (oracle/hybrid_case.py).  Gates:
   * the reference's own: per output row, bf16 relative L2 error <= 0.01 against the FP64 checker
     (:366-378), and exact zeros on identically zero rows (:369-371) -- with the checker using the
-    block_fp8_oracle scale rule this build implements (the test's TPC chain rounds its group scale
+    block_fp8_oracle scale rule the library implements (the test's TPC chain rounds its group scale
     differently, which flips an occasional code);
-  * this build's GEMM gate against oracle/block_fp8.reference, both modes, row-major and packed weights.
+  * the library's GEMM gate against oracle/block_fp8.reference, both modes, row-major and packed weights.
 The chunked case (:389) splits K across calls of the reference's FP16 chain; one call covers it here
 (its activations equal the first case's), run on a padded-stride view of x instead.
 """
